@@ -607,9 +607,10 @@ int lc_hip_trace_get_ray_sort(uint64_t device, int kind, int *enable);
    (segments 1) or from a segment of the queue per XCD (segments 8). */
 int lc_hip_trace_set_fetch(uint64_t device, int kind, uint32_t chunk, uint32_t segments);
 int lc_hip_trace_get_fetch(uint64_t device, int kind, uint32_t *chunk, uint32_t *segments);
-/* Traversal step policy: closest hit takes a triangle step when 4 x (lanes holding triangles) >=
-   tri_quarters x (live lanes), tri_quarters in 1..4 (default 2); a wave stops stepping early to
-   refill once fewer than refill_below of its 64 lanes hold a ray (0 = off, the default). */
+/* Traversal step policy: a wave tests triangles first once its queue of them fills tri_quarters
+   quarters of its 64 lanes, tri_quarters in 1..4 (default 3), and before that whenever more lanes
+   can test one than can visit a node; it stops stepping early to refill once fewer than
+   refill_below of its lanes hold a ray (0 = off; 48 for closest hit and 44 for any hit by default). */
 int lc_hip_trace_set_steps(uint64_t device, int kind, uint32_t tri_quarters, uint32_t refill_below);
 int lc_hip_trace_get_steps(uint64_t device, int kind, uint32_t *tri_quarters, uint32_t *refill_below);
 /* Build knob: 1 = also open multi-triangle leaf candidates while a node has free slots. */

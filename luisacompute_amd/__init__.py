@@ -537,8 +537,8 @@ class Device:
         return c.value, s.value
 
     def set_trace_steps(self, kind, tri_quarters, refill_below=0):
-        """Traversal step policy: triangle-step threshold (1..4 quarters of the live lanes) and
-        early refill below that many live lanes (0 off)."""
+        """Traversal step policy: queued triangles are tested first once they fill this many quarters
+        (1..4) of a wave; early refill below that many live lanes (0 off)."""
         _check(lib().lc_hip_trace_set_steps(self.handle, 1 if kind == "any" else 0, tri_quarters, refill_below),
                "set_trace_steps")
 

@@ -5,10 +5,9 @@ Stages (each on the best configuration of the stages before it):
   1. traversal, per trace kind (closest / any) on the 16.7M-triangle soup, searched jointly: block
      size, LDS stack depth, steps between ray refills, sorted or unsorted queue, and how the launch
      hands out queue slots (slots per claim, one queue or a segment per XCD);
-  1b. the traversal step policy on the best stage-1 launch shape and hand-out: the share of live
-     lanes that must hold triangles for a closest-hit wave to take a triangle step (1..3 quarters),
-     the early refill of waves whose live lanes fall below a count (off, 32, 48), and the steps
-     between refills again;
+  1b. the traversal step policy on the best stage-1 launch shape and hand-out: the quarters of a
+     wave that queued triangles fill when they are tested first (1..4), the early refill of waves
+     whose busy lanes fall below a count (off, 32, 44, 52), and the steps between refills again;
   2. BVH width (children per wide node, 4 / 6 / 8) on the soup step it serves: BLAS build +
      closest-hit trace;
   3. the wavefront path tracer on the box room: samples per wave (queue chunking), the fetch of its
@@ -36,8 +35,8 @@ STEPS = (8, 16, 32, 128)
 BLOCKS_PER_CU = (0,)
 SORT = (False, True)
 FETCH = ((0, 1), (64, 1), (256, 1), (64, 8), (256, 8))  # (slots per claim, queue segments)
-TRI_QUARTERS = (1, 2, 3)
-REFILL_BELOW = (0, 32, 48)
+TRI_QUARTERS = (1, 2, 3, 4)
+REFILL_BELOW = (0, 32, 44, 52)
 WIDTHS = (4, 6, 8)
 PT_CHUNKS = (0, 2, 4, 8, 16)        # samples per wave (0: about 32M paths per wave)
 PT_FETCH = ((0, 1), (64, 8), (128, 8), (256, 8))
@@ -128,14 +127,13 @@ def tune(device, stream, accel, ray_buffer, hit_buffer, any_buffer, count, repea
 
 
 def tune_steps(device, stream, accel, ray_buffer, hit_buffer, any_buffer, count, result, repeats=3, log=print):
-    """Stage 1b: the step policy on the best stage-1 configuration of each kind (the triangle-step
-    threshold applies to closest hit only)."""
+    """Stage 1b: the step policy on the best stage-1 configuration of each kind."""
     for kind, buf in (("closest", hit_buffer), ("any", any_buffer)):
         fn = (lambda: accel.trace_closest(stream, ray_buffer, buf, count)) if kind == "closest" else \
              (lambda: accel.trace_any(stream, ray_buffer, buf, count))
         c = result[kind]
         timed = []
-        for tq, rb, steps in itertools.product(TRI_QUARTERS if kind == "closest" else (2,), REFILL_BELOW, STEPS):
+        for tq, rb, steps in itertools.product(TRI_QUARTERS, REFILL_BELOW, STEPS):
             device.set_trace_config(kind, c["block"], c["lds_stack"], steps, c["blocks_per_cu"])
             device.set_trace_steps(kind, tq, rb)
             ms = _time(device, stream, fn, "trace_" + kind, repeats)

@@ -85,8 +85,8 @@ struct TraceParams {
     uint32_t hit_record;  // closest hits carry the leaf record index in their padding word
     uint32_t fetch_chunk;    // queue slots a wave claims per atomic (0: exactly what its idle lanes need)
     uint32_t fetch_segments; // 1: one queue counter; kFetchSegments: one segment + counter per XCD
-    uint32_t tri_quarters;   // closest hit: a step tests triangles when 4 x (lanes holding some) >=
-                             // tri_quarters x (live lanes)
+    uint32_t tri_quarters;   // queued triangles are tested first once they fill this many quarters of a
+                             // wave
     uint32_t refill_below;   // a wave stops its steps early to refill once fewer lanes than this
                              // hold a ray (0: refill only after `steps` steps)
 };
@@ -263,16 +263,18 @@ hipError_t trace_launch(const TraceParams &P, hipStream_t stream, bool any, bool
                         int slds);
 
 // ---- host objects ----
+// Launch shape and step policy of a trace kind; the initial values are the tuned ones of the
+// 16.7M-triangle soup (one wave per workgroup: its LDS, 6,400 B, lets 6 run on each SIMD).
 struct TraceConfig {
-    int block = 256;
-    int slds = 16;
+    int block = 64;
+    int slds = 8;
     int steps = 32;
     int blocks_per_cu = 0; // 0: occupancy limit
     bool sort_rays = false; // traverse a queue sorted by origin Morton code + direction octant
-    uint32_t fetch_chunk = 0;    // see TraceParams
-    uint32_t fetch_segments = 1;
-    uint32_t tri_quarters = 2;   // see TraceParams
-    uint32_t refill_below = 0;
+    uint32_t fetch_chunk = 64;   // see TraceParams
+    uint32_t fetch_segments = kFetchSegments;
+    uint32_t tri_quarters = 3;   // see TraceParams
+    uint32_t refill_below = 48;
 };
 
 struct TimingStat {

@@ -421,8 +421,7 @@ uint64_t lc_hip_device_create(int32_t index) {
     }
     if (const char *v = std::getenv("LUISA_HIP_BVH_SAH")) dev->sah_refine = std::atoi(v) != 0 ? 1u : 0u;
     if (const char *v = std::getenv("LUISA_HIP_BVH_WIDTH")) dev->bvh_width = (uint32_t)std::min(8, std::max(2, std::atoi(v)));
-    dev->cfg[0] = TraceConfig{256, 16, 32, 0};
-    dev->cfg[1] = TraceConfig{256, 16, 32, 0};
+    dev->cfg[1].refill_below = 44; // any hit
     if (hipEventCreateWithFlags(&dev->arena_done, hipEventDisableTiming) != hipSuccess) {
         hipFree(dev->error);
         fail(LC_HIP_ERROR_HIP, "device event creation failed");
@@ -2317,9 +2316,9 @@ int lc_hip_trace_set_fetch(uint64_t device, int kind, uint32_t chunk, uint32_t s
     return LC_HIP_OK;
 }
 
-// Traversal step policy of a trace kind (autotuned): the triangle-step threshold of closest-hit
-// traversal (4 x lanes holding triangles >= tri_quarters x live lanes, 1..4) and the early refill
-// (a wave refills once fewer than refill_below of its 64 lanes hold a ray; 0 off).
+// Traversal step policy of a trace kind (autotuned): the quarters of a wave (1..4) that queued
+// triangles fill when they are tested first, and the early refill (a wave refills once fewer than
+// refill_below of its 64 lanes hold a ray; 0 off).
 int lc_hip_trace_set_steps(uint64_t device, int kind, uint32_t tri_quarters, uint32_t refill_below) {
     Device *dev = obj<Device>(device);
     if (!dev || kind < 0 || kind > 1) return fail(LC_HIP_ERROR_INVALID_ARGUMENT, "bad trace kind");

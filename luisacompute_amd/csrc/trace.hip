@@ -21,7 +21,7 @@
 
 #include "lc_hip_bvh.h"
 #include "lc_hip_internal.h"
-#include "traverse.h"
+#include "wave_walker.h"
 
 // Working memory of lc_hip_accel_trace_closest_noalloc: the launch's slot counters, error word
 // and stats in the first kNoAllocWordsBytes, then the per-lane stack spill area. Each GPU holds
@@ -60,15 +60,14 @@ hipError_t noalloc_scratch_lookup(void **device_ptr) {
 // (closest-hit, <= 80 VGPRs) waves per SIMD without spilling; the hint keeps the register
 // allocator there (deeper LDS stacks are limited by LDS first).
 template<bool ANY, bool TWO, bool COUNT, int BLOCK, int SLDS>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu((!TWO && SLDS == 8) ? (ANY ? 7 : 6) : 1)))
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(SLDS == 8 ? (TWO ? 5 : 6) : 1)))
 void k_trace(const TraceParams P) {
-    __shared__ uint2 stk[SLDS > 0 ? SLDS : 1][BLOCK];
+    __shared__ trav::WaveShared<ANY, BLOCK, SLDS> shared;
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u;
-    const uint64_t glane = (uint64_t)blockIdx.x * BLOCK + tid;
     const uint32_t count = P.count_ptr ? min(*P.count_ptr, P.count) : P.count;
-    trav::Walker<ANY, TWO, COUNT, BLOCK, SLDS> W;
-    W.init(P.geo, stk, tid, P.spill + glane * (uint64_t)P.spill_depth, P.spill_depth, P.error);
+    trav::WaveWalker<ANY, TWO, COUNT, BLOCK, SLDS> W;
+    W.init(P, &shared, tid);
 
     // Fetching: the queue is split into kFetchSegments contiguous segments, one per XCD
     // (workgroups are dealt to the XCDs round-robin, so block b runs on XCD b mod 8), each with a
@@ -88,8 +87,6 @@ void k_trace(const TraceParams P) {
     bool drained = false;            // wave-uniform: every segment is used up
     bool active = false, exhausted = false;
     uint64_t rounds = 0; // counting form: refill rounds of this wave
-    uint32_t ray_id = 0; // index within the batch
-    uint32_t batch = 0;  // batch of the current ray
     for (;;) {
         const uint64_t need = __ballot(!active && !exhausted);
         if (need) {
@@ -138,11 +135,8 @@ void k_trace(const TraceParams P) {
             if (!active && !exhausted) {
                 if (my < count) {
                     const uint32_t q = P.order ? P.order[my] : my; // sorted queue: fetch in key order
-                    batch = find_batch(P.batches, q);
-                    ray_id = q - P.batches.b[batch].start;
-                    const float4 *rays = P.batches.b[batch].rays;
-                    const float4 r0 = rays[2 * (uint64_t)ray_id], r1 = rays[2 * (uint64_t)ray_id + 1];
-                    W.start(P.geo, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w, P.batches.b[batch].mask);
+                    const uint32_t b = find_batch(P.batches, q);
+                    W.start(P, b, q - P.batches.b[b].start);
                     active = true;
                 } else if (drained) {
                     exhausted = true; // no slot left in any segment (else: retry next round)
@@ -151,15 +145,9 @@ void k_trace(const TraceParams P) {
         }
         if (!__any(active)) break;
         if (COUNT && lane == (uint32_t)__ffsll((long long)__ballot(1)) - 1u) rounds++;
-        if (active && W.run(P.geo, P.steps, P.tri_quarters, P.refill_below, !drained)) {
-            // the counting form has no output buffers (out is null)
-            if (COUNT) {
-            } else if (ANY) {
-                static_cast<uint8_t *>(P.batches.b[batch].out)[ray_id] = W.any_hit ? 1u : 0u;
-            } else {
-                W.write_hit(reinterpret_cast<uint2 *>(static_cast<char *>(P.batches.b[batch].out) + 24ull * ray_id),
-                            P.hit_record != 0u);
-            }
+        W.run(P, active, !drained);
+        if (active && W.finished()) {
+            if (!COUNT) W.write(P); // the counting form has no output buffers (out is null)
             active = false;
         }
     }
