@@ -89,6 +89,8 @@ struct TraceParams {
                              // wave
     uint32_t refill_below;   // a wave stops its steps early to refill once fewer lanes than this
                              // hold a ray (0: refill only after `steps` steps)
+    uint32_t lanes;          // 0: waves claim slots as they go; else wave w takes the `lanes` slots from
+                             // w x lanes on, and no others (trace_grid)
 };
 
 // ---- kernels (radix.hip) ----
@@ -113,6 +115,16 @@ hipError_t exclusive_scan_u32_counted(hipStream_t stream, const uint32_t *in, ui
                                       uint32_t div);
 
 // ---- kernels (raysort.hip) ----
+// Rays below which a queue is traced in its own order: at 262,144 rays (soups of 1M and 8M
+// triangles, incoherent rays) the sort costs what it saves (370 us either way, 532 before the launch
+// itself got faster); at 131,072 281 us sorted against 241, at 524,288 565 against 668.
+constexpr uint64_t kSortMinRays = 1u << 18;
+// Two-level scenes whose rays' queues are sorted: those where a point lies in this many instance boxes
+// on average. Where instances lie apart, few of a ray's fetches are those of its neighbours in origin
+// and direction (2.1M rays, unsorted / sorted: 2 overlapping soups of 1M triangles 3,763 / 3,145 us, 8
+// of them 5,825 / 5,075; 64 side by side 3,046 / 3,283, 1,000 spheres side by side 1,626 / 1,688; 1,024
+// scattered instances 757 / 885).
+constexpr double kSortMinOverlap = 1.5;
 // count_ptr (device word, may be null): only the first min(*count_ptr, n) rays are sorted.
 size_t ray_sort_scratch_bytes(uint32_t n);
 hipError_t ray_sort(hipStream_t stream, const BatchTable &batches, uint32_t n, const uint32_t *count_ptr,
@@ -259,6 +271,13 @@ int trace_blocks_per_cu(bool any, bool two, bool count, int block, int slds);
 constexpr size_t kNoAllocScratchBytes = 32ull << 20;
 constexpr size_t kNoAllocWordsBytes = 4096; // slot counters, error word, stats; the spill area follows
 hipError_t noalloc_scratch_lookup(void **device_ptr);
+// Workgroups and rays per wave (TraceParams::lanes) of a launch over at most `count` rays; at most
+// blocks_per_cu workgroups run on each of `cu_count` CUs.
+struct TraceGrid {
+    int grid;
+    uint32_t lanes;
+};
+TraceGrid trace_grid(uint64_t count, int block, int blocks_per_cu, int cu_count);
 hipError_t trace_launch(const TraceParams &P, hipStream_t stream, bool any, bool two, bool count, int grid, int block,
                         int slds);
 
@@ -460,6 +479,7 @@ struct Accel {
     bool built = false;
     uint32_t max_blas_depth = 0;
     float world_bounds[6] = {0, 0, 0, 0, 0, 0}; // union of instance world boxes (ray-sort keys)
+    double box_overlap = 0.0; // instance boxes that cover a point of the scene box on average (last build)
     // device-side instance table for the in-kernel instance ops (state[count] is the
     // out-of-range-index flag word); written at every build, folded back into `inst` before the
     // next build when instance writes were issued

@@ -1425,6 +1425,7 @@ int lc_hip_accel_build(uint64_t device, uint64_t stream, uint64_t accel, uint32_
     // world boxes of instances: 8 transformed BLAS-box corners, padded by a relative epsilon
     float *boxes = reinterpret_cast<float *>(a->stage + off_box);
     {
+        double volumes = 0.0;
         float wlo[3] = {3e38f, 3e38f, 3e38f}, whi[3] = {-3e38f, -3e38f, -3e38f};
         for (uint32_t i = 0; i < instance_count; i++) {
             float lo[3] = {3e38f, 3e38f, 3e38f}, hi[3] = {-3e38f, -3e38f, -3e38f};
@@ -1443,6 +1444,7 @@ int lc_hip_accel_build(uint64_t device, uint64_t stream, uint64_t accel, uint32_
                     wlo[k] = std::min(wlo[k], lo[k]);
                     whi[k] = std::max(whi[k], hi[k]);
                 }
+                volumes += ((double)hi[0] - lo[0]) * ((double)hi[1] - lo[1]) * ((double)hi[2] - lo[2]);
             } else {
                 // no geometry: a degenerate box far outside any scene (never entered: blas_nodes == 0)
                 for (int k = 0; k < 3; k++) { lo[k] = hi[k] = 3e38f; }
@@ -1455,6 +1457,9 @@ int lc_hip_accel_build(uint64_t device, uint64_t stream, uint64_t accel, uint32_
             a->world_bounds[k] = wlo[k] <= whi[k] ? wlo[k] : 0.0f;
             a->world_bounds[3 + k] = wlo[k] <= whi[k] ? whi[k] : 0.0f;
         }
+        double volume = 1.0;
+        for (int k = 0; k < 3; k++) volume *= (double)a->world_bounds[3 + k] - a->world_bounds[k];
+        a->box_overlap = volume > 0.0 ? volumes / volume : 0.0;
     }
     if (instance_count > 1) {
         p = a->boxes; cap = a->box_cap;
@@ -1689,8 +1694,9 @@ static int trace_launch_batches(Device *dev, Accel *a, hipStream_t s, const lc_h
     const TraceConfig &cfg = dev->cfg[any ? 1 : 0];
     // the counting form runs the timed form's grid (same waves, same queue hand-out)
     int bpc = cfg.blocks_per_cu > 0 ? cfg.blocks_per_cu : trace_blocks_per_cu(any, two, false, cfg.block, cfg.slds);
-    uint64_t want = (total + cfg.block - 1) / cfg.block;
-    int grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)bpc * dev->cu_count, want));
+    const TraceGrid tg = trace_grid(total, cfg.block, bpc, dev->cu_count);
+    const int grid = tg.grid;
+    P.lanes = tg.lanes;
     P.spill_depth = stack_need > (uint32_t)cfg.slds ? stack_need - (uint32_t)cfg.slds : 0u;
     size_t spill_bytes = (size_t)grid * cfg.block * P.spill_depth * sizeof(uint2);
     StreamScratch *S = stream_scratch(dev, s);
@@ -1708,10 +1714,12 @@ static int trace_launch_batches(Device *dev, Accel *a, hipStream_t s, const lc_h
     if (counting) LC_HIP_TRY(hipMemsetAsync(S->stats, 0, 5 * sizeof(unsigned long long), s));
     // per-ray results do not depend on the order; the counting form traverses the same sorted
     // queue as the timed form, so its node / triangle totals describe that launch. Queues counted
-    // on the device sort their first *count_ptr rays (the sort reads the count when it runs). A
+    // on the device sort their first *count_ptr rays (the sort reads the count when it runs).
+    // Launches of fewer than kSortMinRays rays, and those over instances that lie apart
+    // (kSortMinOverlap), are traced in queue order. A
     // captured launch sorts when the stream already holds the sort's working memory (captures
     // cannot allocate) and otherwise traces the queue in its own order.
-    bool sort = cfg.sort_rays && total > 1 && !P.geo.empty;
+    bool sort = cfg.sort_rays && total >= kSortMinRays && !P.geo.empty && (!two || a->box_overlap >= kSortMinOverlap);
     if (sort && capturing(s) && S->sort_bytes < ray_sort_scratch_bytes(P.count)) sort = false;
     if (sort) LC_HIP_GROW((S, s, S->sort, S->sort_bytes, ray_sort_scratch_bytes(P.count)));
     {
@@ -1933,8 +1941,8 @@ int lc_hip_accel_trace_closest_noalloc(uint64_t device, uint64_t stream, uint64_
     std::lock_guard<std::mutex> dl(dev->mu);
     const TraceConfig &cfg = dev->cfg[0];
     const int bpc = cfg.blocks_per_cu > 0 ? cfg.blocks_per_cu : trace_blocks_per_cu(false, two, false, cfg.block, cfg.slds);
-    const uint64_t want = ((uint64_t)ray_count + cfg.block - 1) / cfg.block;
-    uint64_t grid = std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)bpc * dev->cu_count, want));
+    TraceGrid tg = trace_grid(ray_count, cfg.block, bpc, dev->cu_count);
+    uint64_t grid = (uint64_t)tg.grid;
     P.spill_depth = stack_need > (uint32_t)cfg.slds ? stack_need - (uint32_t)cfg.slds : 0u;
     const size_t spill_per_block = (size_t)cfg.block * P.spill_depth * sizeof(uint2);
     const size_t spill_cap = kNoAllocScratchBytes - kNoAllocWordsBytes;
@@ -1942,7 +1950,11 @@ int lc_hip_accel_trace_closest_noalloc(uint64_t device, uint64_t stream, uint64_
         return fail(LC_HIP_ERROR_UNSUPPORTED, "traversal stacks of one workgroup need " + std::to_string(spill_per_block) +
                                                   " spill bytes, more than the no-allocation scratch holds (" +
                                                   std::to_string(spill_cap) + ")");
-    if (spill_per_block) grid = std::min<uint64_t>(grid, spill_cap / spill_per_block);
+    if (spill_per_block && grid > spill_cap / spill_per_block) { // a smaller grid: waves claim slots as they go
+        grid = spill_cap / spill_per_block;
+        tg.lanes = 0u;
+    }
+    P.lanes = tg.lanes;
     static_assert(576 + 2 * sizeof(unsigned long long) <= kNoAllocWordsBytes, "no-allocation words");
     char *base = static_cast<char *>(dev->noalloc_scratch);
     P.ray_counter = reinterpret_cast<uint32_t *>(base);

@@ -14,6 +14,7 @@
 // read from device memory (`count_ptr`) for launches whose queue length is produced on the GPU.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cfloat>
 #include <cstdint>
 #include <map>
@@ -86,6 +87,21 @@ void k_trace(const TraceParams P) {
     uint32_t pool = 0, pool_end = 0; // wave-uniform: unclaimed slots [pool, pool_end)
     bool drained = false;            // wave-uniform: every segment is used up
     bool active = false, exhausted = false;
+    if (P.lanes != 0u) {
+        // every ray has a lane: wave w takes the slots [w lanes, w lanes + lanes) of the queue, with
+        // w counted XCD by XCD (block b runs on XCD b mod 8), so that each XCD has its own part
+        const uint32_t per_xcd = gridDim.x / kFetchSegments;
+        const uint32_t b = (blockIdx.x % kFetchSegments) * per_xcd + blockIdx.x / kFetchSegments;
+        const uint64_t w = (uint64_t)b * (BLOCK / 64) + (tid >> 6);
+        const uint64_t my = w * P.lanes + lane;
+        drained = exhausted = true;
+        if (lane < P.lanes && my < count) {
+            const uint32_t q = P.order ? P.order[my] : (uint32_t)my;
+            const uint32_t bt = find_batch(P.batches, q);
+            W.start(P, bt, q - P.batches.b[bt].start);
+            active = true;
+        }
+    }
     uint64_t rounds = 0; // counting form: refill rounds of this wave
     for (;;) {
         const uint64_t need = __ballot(!active && !exhausted);
@@ -218,9 +234,29 @@ int trace_blocks_per_cu(bool any, bool two, bool count, int block, int slds) {
     return count ? occupancy_cfg<false, false, true>(block, slds) : occupancy_cfg<false, false, false>(block, slds);
 }
 
+// A launch whose rays all fit the lanes that can be resident hands them out once, without slot
+// counters (and without the launch that clears them). When that leaves SIMDs without a wave, waves
+// take fewer rays instead, down to kMinLanes: a wave lasts as long as its slowest ray plus the
+// triangle steps of the others, one step after another, each a memory latency (4,096 rays on
+// 81,920 triangles: 98 us with 64 rays per wave, 60 with 4; 16 per wave 65).
+TraceGrid trace_grid(uint64_t count, int block, int blocks_per_cu, int cu_count) {
+    constexpr uint32_t kMinLanes = 4;
+    const uint64_t cus = (uint64_t)std::max(1, cu_count);
+    const uint64_t most = (uint64_t)std::max(1, blocks_per_cu) * cus;
+    const uint64_t waves_per_block = (uint64_t)(block / 64);
+    if (count > most / kFetchSegments * kFetchSegments * (uint64_t)block) return {(int)most, 0u};
+    const uint64_t simds = 4u * cus;
+    uint32_t lanes = kMinLanes;
+    while (lanes < 64u && (count + lanes - 1) / lanes > simds) lanes *= 2u;
+    uint64_t grid = ((count + lanes - 1) / lanes + waves_per_block - 1) / waves_per_block;
+    grid = (grid + kFetchSegments - 1) / kFetchSegments * kFetchSegments; // k_trace counts waves XCD by XCD
+    return {(int)grid, lanes};
+}
+
 hipError_t trace_launch(const TraceParams &P, hipStream_t stream, bool any, bool two, bool count, int grid, int block,
                         int slds) {
-    hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, stream, P.ray_counter);
+    if (P.lanes == 0u)
+        hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, stream, P.ray_counter);
     if (any) {
         if (two) return count ? launch_cfg<true, true, true>(P, stream, grid, block, slds) : launch_cfg<true, true, false>(P, stream, grid, block, slds);
         return count ? launch_cfg<true, false, true>(P, stream, grid, block, slds) : launch_cfg<true, false, false>(P, stream, grid, block, slds);

@@ -82,7 +82,7 @@ struct WaveWalker {
     float tmin, tmax;
     uint32_t batch, ray;   // which ray this is: its batch and the index there
     float t_best;          // nearest hit so far (inside an instance: or the limit it was entered with)
-    bool any_hit;
+    bool any_hit;          // some hit so far (two-level closest hit: in an instance left before)
     uint32_t g_base, g_mask, t_base, t_mask;
     int floor;             // stack height of the current level: 0, or where the instance was entered
     uint32_t cur_inst;     // instance this lane is in (two-level; kWorld: in the TLAS)
@@ -157,7 +157,6 @@ struct WaveWalker {
             nodes = G.tlas_nodes;
             ray_setup(R);
             g_mask = G.empty ? 0u : ((1u << R.oct) | (1u << 8));
-            if (!ANY && !COUNT) store_hit(P, kMissKey, 0u); // the nearest hit of the instances left so far: none
         } else {
             xform_point(G.inst_inv, o, R.o);
             xform_vector(G.inst_inv, d, R.d);
@@ -272,10 +271,15 @@ struct WaveWalker {
                     if (COUNT) {
                         t_best = t_value((uint32_t)(k >> 32));
                     } else {
-                        const uint2 *h = out_hit(P);
-                        const uint2 h0 = h[0];
-                        const float t = t_value((uint32_t)(k >> 32)), t0 = __uint_as_float(h[2].x);
-                        if (h0.y == 0xFFFFFFFFu || nearer(t, cur_inst, prim, t0, h0.x, h0.y)) store_hit(P, k, cur_inst);
+                        const float t = t_value((uint32_t)(k >> 32));
+                        bool better = !any_hit;
+                        if (any_hit) {
+                            const uint2 *h = out_hit(P);
+                            const uint2 h0 = h[0];
+                            better = nearer(t, cur_inst, prim, __uint_as_float(h[2].x), h0.x, h0.y);
+                        }
+                        if (better) store_hit(P, k, cur_inst);
+                        any_hit = true;
                         t_best = t;
                     }
                 }
@@ -371,6 +375,12 @@ struct WaveWalker {
         t_mask = nt;
     }
 
+    // Counting form: a step of the wave, in which this lane is busy or not.
+    __device__ __forceinline__ void account(bool busy) {
+        if (busy) n_live++;
+        if (lane == 0u) n_wave++;
+    }
+
     // Runs up to P.steps steps of the wave's rays (`active` lanes hold one), each of the kind that
     // the most lanes can take: a triangle step tests one queued pair per lane, an instance step
     // moves lanes into and out of instances, a node step visits a node per lane. A queue that fills
@@ -388,15 +398,11 @@ struct WaveWalker {
             if ((uint32_t)__popcll(wm) < refill_below &&
                 (uint32_t)__popcll(__ballot(active && !finished())) < refill_below)
                 return;
-            if (COUNT) {
-                const bool testing = (queued >= full || (wm == 0ull && queued != 0u)) && lane < min(64u, queued);
-                if ((active && !finished()) || testing) n_live++;
-                if (lane == 0u) n_wave++;
-            }
             bool tri = queued >= full || (queued != 0u && queued >= (uint32_t)__popcll(wm));
             if (TWO && !tri) {
                 const uint64_t im = __ballot(active && inst_work());
                 if (im != 0ull && (wm == 0ull || (uint32_t)__popcll(im) >= (uint32_t)__popcll(wm))) {
+                    if (COUNT) account(active && !finished());
                     if (active && inst_work()) instance_step(P);
                     continue;
                 }
@@ -405,6 +411,7 @@ struct WaveWalker {
                 if (queued == 0u) return; // every ray is done
                 tri = true;
             }
+            if (COUNT) account((active && !finished()) || (tri && lane < queued));
             if (tri) triangle_step();
             else if (work) visit(P);
             queue_triangles(active);
@@ -430,10 +437,11 @@ struct WaveWalker {
         }
     }
 
-    // The result of a finished ray (two-level closest hits are written as instances are left).
+    // The result of a finished ray (two-level closest hits were written as instances were left).
     __device__ __forceinline__ void write(const TraceParams &P) const {
         if (ANY) static_cast<uint8_t *>(P.batches.b[batch].out)[ray] = any_hit ? 1u : 0u;
         else if (!TWO) store_hit(P, sh->key[tid], 0u);
+        else if (!any_hit) store_hit(P, kMissKey, 0u);
     }
 };
 
