@@ -13,6 +13,7 @@
 // can be recorded into a graph with the grid sized for the capacity. Values may be the identity
 // (`vals_in` null): the first pass then writes each item's input index.
 // Traffic per pass and item: 4 B read (upsweep) + 8 B read and 8 B written (downsweep).
+// Sorts of at most 8,192 items run in one workgroup instead (k_rs_small).
 //
 // Scan: exclusive prefix sum of up to 2^32-1 uint32 words by one workgroup of 1,024 threads
 // (16,384 words per round); the lists it serves (per-workgroup counts of the build phases) are
@@ -253,6 +254,95 @@ __global__ __launch_bounds__(kRsBlock) void k_rs_downsweep(const uint32_t *keys_
     }
 }
 
+// All passes of a sort of at most kSmallBlock x ITEMS items by one workgroup, keys and values in
+// registers between them: ranking as in k_rs_downsweep, the exchange through LDS. Three kernels per
+// pass over one or two tiles take their latencies one after another: the 12 launches of a build's
+// 30-bit sort of 5,120 keys 84 us, this 28.
+constexpr int kSmallBlock = 1024;
+constexpr int kSmallItems = 8; // most items per thread
+constexpr int kSmallWaves = kSmallBlock / 64;
+
+template<int ITEMS>
+__global__ __launch_bounds__(kSmallBlock) void k_rs_small(const uint32_t *keys_in, const uint32_t *vals_in,
+                                                          uint32_t *keys_out, uint32_t *vals_out, uint32_t cap,
+                                                          const uint32_t *count_ptr, uint32_t begin_bit,
+                                                          uint32_t end_bit) {
+    __shared__ uint32_t s_hist[kSmallWaves][256]; // per-wave digit counters, then offsets
+    __shared__ uint32_t s_buf[kSmallBlock * ITEMS];
+    __shared__ uint32_t s_wave[kSmallWaves];
+    const uint32_t t = threadIdx.x, w = t >> 6, lane = t & 63u;
+    const uint32_t n = item_count(count_ptr, cap);
+    const uint32_t base = w * 64u * ITEMS + lane;
+    uint32_t key[ITEMS], val[ITEMS], pos[ITEMS];
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+        const uint32_t i = base + j * 64u;
+        key[j] = i < n ? keys_in[i] : 0u;
+        val[j] = i < n ? (vals_in ? vals_in[i] : i) : 0u;
+    }
+    for (uint32_t shift = begin_bit; shift < end_bit; shift += 8u) {
+        const uint32_t mask = end_bit - shift < 8u ? (1u << (end_bit - shift)) - 1u : 0xFFu;
+#pragma unroll
+        for (int k = 0; k < kSmallWaves * 256 / kSmallBlock; k++) (&s_hist[0][0])[k * kSmallBlock + t] = 0u;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) {
+            const bool valid = base + j * 64u < n;
+            const uint64_t act = __ballot(valid);
+            if (act == 0) break;
+            const uint32_t d = (key[j] >> shift) & mask;
+            const uint64_t m = match_digit(d, act);
+            const uint32_t before = valid ? s_hist[w][d] : 0u;
+            pos[j] = before + lanes_below(m);
+            if (valid && lane == (uint32_t)__builtin_ctzll(m)) s_hist[w][d] = before + (uint32_t)__popcll(m);
+        }
+        __syncthreads();
+        uint32_t run = 0; // digit t: offsets of the waves' items within the digit
+        if (t < 256u) {
+#pragma unroll
+            for (int k = 0; k < kSmallWaves; k++) {
+                const uint32_t c = s_hist[k][t];
+                s_hist[k][t] = run;
+                run += c;
+            }
+        }
+        uint32_t all;
+        const uint32_t start = block_exclusive_scan<kSmallBlock>(run, all, s_wave); // synchronises
+        if (t < 256u) {
+#pragma unroll
+            for (int k = 0; k < kSmallWaves; k++) s_hist[k][t] += start;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++) {
+            if (base + j * 64u < n) {
+                pos[j] += s_hist[w][(key[j] >> shift) & mask];
+                s_buf[pos[j]] = key[j];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++)
+            if (base + j * 64u < n) key[j] = s_buf[base + j * 64u];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++)
+            if (base + j * 64u < n) s_buf[pos[j]] = val[j];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < ITEMS; j++)
+            if (base + j * 64u < n) val[j] = s_buf[base + j * 64u];
+    }
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+        const uint32_t i = base + j * 64u;
+        if (i < n) {
+            keys_out[i] = key[j];
+            vals_out[i] = val[j];
+        }
+    }
+}
+
 // count_ptr != null: n = ceil(*count_ptr / div) (a list's chunk count, known on the device only).
 __global__ __launch_bounds__(kScanBlock) void k_exclusive_scan(const uint32_t *in, uint32_t *out, uint32_t n,
                                                                const uint32_t *count_ptr, uint32_t div) {
@@ -312,6 +402,13 @@ hipError_t radix_sort_pairs_with(hipStream_t stream, void *count_temp, size_t co
     if ((reinterpret_cast<uintptr_t>(keys_in) | reinterpret_cast<uintptr_t>(keys_out) |
          reinterpret_cast<uintptr_t>(alt_k)) % 16 != 0)
         return hipErrorInvalidValue;
+    if (cap <= (uint32_t)(kSmallBlock * kSmallItems)) {
+        const auto small = cap <= kSmallBlock ? k_rs_small<1> : (cap <= 2 * kSmallBlock ? k_rs_small<2>
+                           : (cap <= 4 * kSmallBlock ? k_rs_small<4> : k_rs_small<8>));
+        hipLaunchKernelGGL(small, dim3(1), dim3(kSmallBlock), 0, stream, keys_in, vals_in, keys_out, vals_out, cap,
+                           count_ptr, begin_bit, end_bit);
+        return hipGetLastError();
+    }
     const uint32_t nt = rs_tiles(cap);
     uint32_t *counts = static_cast<uint32_t *>(count_temp);
     uint32_t *totals = reinterpret_cast<uint32_t *>(static_cast<char *>(count_temp) + align256(256 * (size_t)nt * 4));
