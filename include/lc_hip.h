@@ -616,7 +616,7 @@ int lc_hip_trace_get_steps(uint64_t device, int kind, uint32_t *tri_quarters, ui
 /* Build knob: 1 = also open multi-triangle leaf candidates while a node has free slots. */
 int lc_hip_build_set_split_small(uint64_t device, int enable);
 /* Build knob: SAH refinement of FAST_TRACE builds (the radix tree's clusters of <= 64 primitives
-   rebuilt by binned SAH). 1 = on (the default, unless the environment sets LUISA_HIP_BVH_SAH=0),
+   rebuilt by sweep SAH). 1 = on (the default, unless the environment sets LUISA_HIP_BVH_SAH=0),
    0 = off. FAST_BUILD builds never refine. */
 int lc_hip_build_set_sah(uint64_t device, int enable);
 /* Build knob: children per wide BVH node, 2..8 (default 8, or LUISA_HIP_BVH_WIDTH); the node

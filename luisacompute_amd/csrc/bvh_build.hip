@@ -134,9 +134,10 @@ __device__ __forceinline__ void write_record(const PrimSource &src, uint32_t pri
     hi = make_float3(fmaxf(a.x, fmaxf(b.x, c.x)), fmaxf(a.y, fmaxf(b.y, c.y)), fmaxf(a.z, fmaxf(b.z, c.z)));
 }
 
-__global__ void k_init(BuildCounters *ctr, uint32_t *slots, uint32_t nslots) {
+__global__ void k_init(BuildCounters *ctr, uint32_t *slots, uint32_t nslots, uint32_t *error) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i == 0) {
+        *error = 0u;
         ctr->node_count = 1;
         ctr->tri_count = 0;
         ctr->depth = 0;
@@ -181,8 +182,11 @@ __global__ __launch_bounds__(kBlock) void k_centroid_bounds(PrimSource src, uint
         int a = threadIdx.x;
         float v = part[0][a];
         for (int w = 1; w < kBlock / 64; w++) v = a < 3 ? fminf(v, part[w][a]) : fmaxf(v, part[w][a]);
-        if (a < 3) atomicMin(&ctr->cbounds[a], f2ord(v));
-        else atomicMax(&ctr->cbounds[a], f2ord(v));
+        // six words on one line serialise every workgroup's atomics (85M/s): only those that still move
+        // a bound are issued
+        const int o = f2ord(v), now = __hip_atomic_load(&ctr->cbounds[a], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (a < 3 && o < now) atomicMin(&ctr->cbounds[a], o);
+        if (a >= 3 && o > now) atomicMax(&ctr->cbounds[a], o);
     }
 }
 
@@ -616,7 +620,7 @@ __device__ __forceinline__ uint32_t ord_u32(float f) {
 
 // ---- SAH refinement (FAST_TRACE builds). The radix tree is cut into clusters: the highest
 // nodes with at most kSahCluster primitives (their parent has more). Each cluster's subtree is
-// rebuilt top-down by binned SAH over its primitives (one wave per cluster), and its primitives
+// rebuilt top-down by sweep SAH over its primitives (one wave per cluster), and its primitives
 // are reordered into the new tree's leaf order, so every node still covers a contiguous run of
 // positions and the rest of the build (bottom-up boxes from the cluster roots, collapse) is
 // unchanged. The rebuilt subtree keeps the radix tree's index rule: a node split after position
@@ -625,7 +629,6 @@ __device__ __forceinline__ uint32_t ord_u32(float f) {
 // cluster root keeps its own index (its parent's link is untouched).
 constexpr uint32_t kSahCluster = 64; // primitives per cluster (one per lane of a wave)
 static_assert(kSahCluster == 64, "k_sah_clusters runs one wave64 per workgroup");
-constexpr int kSahBins = 16;         // bins per axis: 15 split candidates per axis, 45 lanes
 
 // Cluster roots in position order: the thread at position `pos` climbs from leaf pos while the
 // parent starts at pos and holds at most kSahCluster primitives; it reports the node it stops at
@@ -657,36 +660,6 @@ __global__ __launch_bounds__(kPhaseBlock) void k_sah_cut(uint32_t n, BinaryTree 
     compact_deferred(found, pend, bcount);
 }
 
-// Wave64 reductions through DPP row operations (VALU lane moves, no LDS round trips): pairs,
-// quads, half rows, rows, then rows 1 / 3 take lane 15 / 47 and rows 2 / 3 lane 31; lane 63 ends
-// with the whole wave's value, broadcast with readlane. Every lane of the wave takes part.
-template<bool MAX, int CTRL, int ROW_MASK>
-__device__ __forceinline__ float dpp_step(float v) {
-    const int o = __builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, ROW_MASK, 0xF, false);
-    return MAX ? fmaxf(v, __int_as_float(o)) : fminf(v, __int_as_float(o));
-}
-template<bool MAX>
-__device__ __forceinline__ float wave_reduce(float v) {
-    v = dpp_step<MAX, 0xB1, 0xF>(v);  // quad_perm [1,0,3,2]
-    v = dpp_step<MAX, 0x4E, 0xF>(v);  // quad_perm [2,3,0,1]
-    v = dpp_step<MAX, 0x141, 0xF>(v); // row_half_mirror
-    v = dpp_step<MAX, 0x140, 0xF>(v); // row_mirror
-    v = dpp_step<MAX, 0x142, 0xA>(v); // row_bcast:15 into rows 1 and 3
-    v = dpp_step<MAX, 0x143, 0xC>(v); // row_bcast:31 into rows 2 and 3
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-}
-__device__ __forceinline__ float wave_sum_min(float v, bool on) { return wave_reduce<false>(on ? v : FLT_MAX); }
-__device__ __forceinline__ float wave_sum_max(float v, bool on) { return wave_reduce<true>(on ? v : -FLT_MAX); }
-__device__ __forceinline__ float lane_value(float v, uint32_t lane) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), (int)lane));
-}
-
-// Bin of a doubled centroid (NaN and values below the first boundary go to bin 0).
-__device__ __forceinline__ int sah_bin(float cv, float cmin, float scale) {
-    const float x = (cv - cmin) * scale;
-    return x >= 1.0f ? min(kSahBins - 1, (int)fminf(x, (float)kSahBins)) : 0;
-}
-
 // Orders the LDS accesses of one wave (LDS operations of a wave complete in order; this keeps the
 // compiler from moving them across the point). Unlike __syncthreads it does not wait for the
 // wave's global stores, so a workgroup of exactly one wave uses it in place of a barrier.
@@ -695,41 +668,63 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// One wave (one workgroup of 64) per cluster, clusters taken in a grid-stride loop. The cluster's
-// primitives sit in LDS in position order (box, doubled centroid, local index) and move when a
-// task is partitioned, so the candidate scans read consecutive LDS words. A task (positions
-// [a, b], node index) is split by the lanes: lane L < 45 scores candidate (axis L / 15, boundary
-// L % 15 + 1) over the task's primitives, the cheapest area(left) * n_left + area(right) * n_right
-// wins (lowest lane on ties), and a stable partition reorders the positions. Tasks of two
-// primitives need no search. Centroids that coincide on every axis are split at the middle.
+struct Box6 {
+    float3 lo, hi;
+};
+__device__ __forceinline__ float lane_float(int lane4, float v) {
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(lane4, __float_as_int(v)));
+}
+// b grown by the box that lane lane4 / 4 holds.
+__device__ __forceinline__ void merge_lane(Box6 &b, int lane4) {
+    b.lo.x = fminf(b.lo.x, lane_float(lane4, b.lo.x));
+    b.lo.y = fminf(b.lo.y, lane_float(lane4, b.lo.y));
+    b.lo.z = fminf(b.lo.z, lane_float(lane4, b.lo.z));
+    b.hi.x = fmaxf(b.hi.x, lane_float(lane4, b.hi.x));
+    b.hi.y = fmaxf(b.hi.y, lane_float(lane4, b.hi.y));
+    b.hi.z = fmaxf(b.hi.z, lane_float(lane4, b.hi.z));
+}
+
+// One wave (one workgroup of 64) per cluster, clusters taken in a grid-stride loop, a whole tree
+// level at a time with one lane per primitive. The cluster is kept as three lists of its primitives,
+// sorted by centroid along x, y and z; a node is a run of positions [a, b], the same in all three.
+// Lane p of a run scores the splits after position p: area(a .. p) * n_left + area(p + 1 .. b) *
+// n_right from an inclusive prefix and suffix of the boxes in each list (merging with a lane's own
+// box again changes nothing, so the lanes at the run's ends need no guard). The run's cheapest split
+// (ties: the one nearest the middle, so that equal boxes halve) marks its right side, and the three
+// lists are partitioned stably by ballots. A level costs the same however many nodes it holds:
+// one task after another over the whole wave, scanning its primitives for 45 binned candidates, took
+// 1,016 us for 1M triangles where this takes 373, and 118 us for 5,120 where this takes 35, for trees
+// that trace alike (1M soup 1,238 and 1,236 us). LDS lane exchanges bound the large builds (12 per
+// doubling, list and direction), the ~8 levels one after another the small ones.
 __global__ __launch_bounds__(64) void k_sah_clusters(const uint32_t *entries, const uint32_t *count_ptr, BinaryTree bt,
                                                      uint32_t *ids, const TriRecord *prec, TriRecord *srec,
                                                      const float4 *pbox) {
     __shared__ float s_box[6][kSahCluster];
-    __shared__ float s_cen[3][kSahCluster];
-    __shared__ uint32_t s_loc[kSahCluster];
-    __shared__ uint32_t s_pos[kSahCluster];
-    __shared__ uint2 s_task[kSahCluster];
-    const uint32_t lane = threadIdx.x;
+    __shared__ uint32_t s_ord[kSahCluster];
+    __shared__ uint32_t s_side[kSahCluster];
+    const int lane = (int)threadIdx.x;
+    const uint64_t lt = (1ull << lane) - 1ull;
     const uint32_t count = *count_ptr;
     for (uint32_t c = blockIdx.x; c < count; c += gridDim.x) {
         const uint32_t ref = entries[c];
         if (ref & kLeafBit) { // a single primitive: its record goes to its position unchanged
             const uint32_t pos = ref & ~kLeafBit;
-            if (srec && lane < 3u) {
+            if (srec && lane < 3) {
                 const float4 *src = reinterpret_cast<const float4 *>(prec + ids[pos]);
                 reinterpret_cast<float4 *>(srec + pos)[lane] = src[lane];
             }
             continue;
         }
         const uint2 rg = bt.range[ref];
-        const uint32_t f = rg.x, m = rg.y - rg.x + 1u; // 2 <= m <= kSahCluster
+        const uint32_t f = rg.x;
+        const int m = (int)(rg.y - rg.x) + 1; // 2 <= m <= kSahCluster
         const bool mine = lane < m;
         uint32_t id = 0;
         float4 r0 = make_float4(0.f, 0.f, 0.f, 0.f), r1 = r0, r2 = r0;
+        uint32_t key[3] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu};
         if (mine) {
             float3 lo, hi;
-            id = ids[f + lane];
+            id = ids[f + (uint32_t)lane];
             if (srec) {
                 const float4 *src = reinterpret_cast<const float4 *>(prec + id);
                 r0 = src[0];
@@ -742,126 +737,103 @@ __global__ __launch_bounds__(64) void k_sah_clusters(const uint32_t *entries, co
             }
             s_box[0][lane] = lo.x; s_box[1][lane] = lo.y; s_box[2][lane] = lo.z;
             s_box[3][lane] = hi.x; s_box[4][lane] = hi.y; s_box[5][lane] = hi.z;
-            s_cen[0][lane] = lo.x + hi.x; s_cen[1][lane] = lo.y + hi.y; s_cen[2][lane] = lo.z + hi.z;
-            s_loc[lane] = lane;
+            // centroids as ordered integers whose low 6 bits are the lane, so no two are equal
+            key[0] = (ord_u32(lo.x + hi.x) & ~63u) | (uint32_t)lane;
+            key[1] = (ord_u32(lo.y + hi.y) & ~63u) | (uint32_t)lane;
+            key[2] = (ord_u32(lo.z + hi.z) & ~63u) | (uint32_t)lane;
         }
-        if (lane == 0u) s_task[0] = make_uint2(m - 1u, ref); // positions [0, m - 1] packed as b, root index
-        wave_sync();
-        int sp = 1;
-        while (sp > 0) { // uniform: every lane pops the same task
-            sp--;
-            const uint2 task = s_task[sp];
-            const uint32_t a = task.x >> 16, b = task.x & 0xFFFFu, idx = task.y;
-            const uint32_t mt = b - a + 1u;
-            // lane j holds the primitive at position a + j
-            const bool on = lane < mt;
-            const uint32_t pj = on ? a + lane : a;
-            const float3 blo = make_float3(s_box[0][pj], s_box[1][pj], s_box[2][pj]);
-            const float3 bhi = make_float3(s_box[3][pj], s_box[4][pj], s_box[5][pj]);
-            const float bc[3] = {s_cen[0][pj], s_cen[1][pj], s_cen[2][pj]};
-            const uint32_t bloc = s_loc[pj];
-            uint32_t nl = 1u;
-            float3 llo, lhi, rlo, rhi;
-            bool by_bins = false;
-            uint32_t best_axis = 0, best_k = 0;
-            float cmin[3] = {0.f, 0.f, 0.f}, cscale[3] = {0.f, 0.f, 0.f};
-            if (mt > 2u) {
-                for (int ax = 0; ax < 3; ax++) {
-                    const float mn = wave_sum_min(bc[ax], on), mx = wave_sum_max(bc[ax], on);
-                    cmin[ax] = mn;
-                    cscale[ax] = mx > mn ? fminf((float)kSahBins / (mx - mn), FLT_MAX) : 0.0f;
+        // rank of each primitive along each axis: the keys below its own
+        uint32_t rank[3] = {0u, 0u, 0u}, ord[3];
+        for (int j = 0; j < m; j++)
+            for (int ax = 0; ax < 3; ax++)
+                rank[ax] += (uint32_t)__builtin_amdgcn_readlane((int)key[ax], j) < key[ax] ? 1u : 0u;
+        for (int ax = 0; ax < 3; ax++) {
+            s_ord[mine ? rank[ax] : (uint32_t)lane] = (uint32_t)lane;
+            wave_sync();
+            ord[ax] = s_ord[lane]; // local index of the primitive at this position
+            wave_sync();
+        }
+        int a = mine ? 0 : lane, b = mine ? m - 1 : lane; // this lane's run
+        uint32_t idx = ref;                               // its node
+        uint64_t slot = ~0ull;                            // where its box goes in bt.cbox (none: the cluster root)
+        while (__ballot(b > a) != 0ull) {
+            const bool on = b > a;
+            float best = FLT_MAX;
+            uint32_t axis = 0u;
+#pragma unroll
+            for (int ax = 0; ax < 3; ax++) {
+                const uint32_t o = ord[ax];
+                Box6 P{make_float3(s_box[0][o], s_box[1][o], s_box[2][o]),
+                       make_float3(s_box[3][o], s_box[4][o], s_box[5][o])};
+                Box6 S = P;
+                for (int d = 1; __ballot(b - a >= d) != 0ull; d <<= 1) {
+                    merge_lane(P, (lane - d >= a ? lane - d : lane) << 2);
+                    merge_lane(S, (lane + d <= b ? lane + d : lane) << 2);
                 }
-                // candidate of this lane: a scan of the task's positions
-                float cost = FLT_MAX;
-                float3 clo = make_float3(FLT_MAX, FLT_MAX, FLT_MAX), chi = make_float3(-FLT_MAX, -FLT_MAX, -FLT_MAX);
-                float3 dlo = clo, dhi = chi;
-                const uint32_t ax = lane / (kSahBins - 1), k = lane % (kSahBins - 1) + 1u;
-                if (lane < 3u * (kSahBins - 1) && cscale[ax] > 0.0f) {
-                    const float *cen = s_cen[ax];
-                    uint32_t cl = 0;
-#pragma unroll 4
-                    for (uint32_t q = a; q <= b; q++) {
-                        const float3 qlo = make_float3(s_box[0][q], s_box[1][q], s_box[2][q]);
-                        const float3 qhi = make_float3(s_box[3][q], s_box[4][q], s_box[5][q]);
-                        if ((uint32_t)sah_bin(cen[q], cmin[ax], cscale[ax]) < k) {
-                            cl++;
-                            clo = make_float3(fminf(clo.x, qlo.x), fminf(clo.y, qlo.y), fminf(clo.z, qlo.z));
-                            chi = make_float3(fmaxf(chi.x, qhi.x), fmaxf(chi.y, qhi.y), fmaxf(chi.z, qhi.z));
-                        } else {
-                            dlo = make_float3(fminf(dlo.x, qlo.x), fminf(dlo.y, qlo.y), fminf(dlo.z, qlo.z));
-                            dhi = make_float3(fmaxf(dhi.x, qhi.x), fmaxf(dhi.y, qhi.y), fmaxf(dhi.z, qhi.z));
-                        }
-                    }
-                    if (cl > 0u && cl < mt)
-                        cost = box_area(clo, chi) * (float)cl + box_area(dlo, dhi) * (float)(mt - cl);
+                if (ax == 0 && on && lane == b && slot != ~0ull) { // the whole run's box
+                    bt.cbox[slot] = make_float4(P.lo.x, P.lo.y, P.lo.z, 0.0f);
+                    bt.cbox[slot + 1] = make_float4(P.hi.x, P.hi.y, P.hi.z, 0.0f);
                 }
-                // cheapest candidate, lowest lane on ties (NaN costs never win)
-                const float best = wave_sum_min(cost == cost ? cost : FLT_MAX, true);
-                const uint64_t at = __ballot(cost == best);
-                const uint32_t win = at ? (uint32_t)__ffsll((long long)at) - 1u : 0u;
-                if (best < FLT_MAX && at != 0u && win < 3u * (kSahBins - 1)) {
-                    by_bins = true;
-                    best_axis = win / (kSahBins - 1);
-                    best_k = win % (kSahBins - 1) + 1u;
-                    llo = make_float3(lane_value(clo.x, win), lane_value(clo.y, win), lane_value(clo.z, win));
-                    lhi = make_float3(lane_value(chi.x, win), lane_value(chi.y, win), lane_value(chi.z, win));
-                    rlo = make_float3(lane_value(dlo.x, win), lane_value(dlo.y, win), lane_value(dlo.z, win));
-                    rhi = make_float3(lane_value(dhi.x, win), lane_value(dhi.y, win), lane_value(dhi.z, win));
+                const float right = lane_float((lane + 1) << 2, box_area(S.lo, S.hi));
+                const float cost = box_area(P.lo, P.hi) * (float)(lane - a + 1) + right * (float)(b - lane);
+                if (lane < b && cost < best) {
+                    best = cost;
+                    axis = (uint32_t)ax;
                 }
             }
-            // partition the task's positions: left = bins below best_k (or the first half)
-            bool left;
-            if (by_bins) {
-                left = sah_bin(bc[best_axis], cmin[best_axis], cscale[best_axis]) < (int)best_k;
-            } else {
-                left = lane < mt / 2u;
+            float low = best; // the run's cheapest cost, complete at its last lane
+            for (int d = 1; __ballot(b - a >= d) != 0ull; d <<= 1)
+                low = fminf(low, lane_float((lane - d >= a ? lane - d : lane) << 2, low));
+            low = lane_float(b << 2, low);
+            const uint64_t run = (b >= 63 ? ~0ull : (1ull << (b + 1)) - 1ull) & ~((1ull << a) - 1ull);
+            const uint64_t at = __ballot(lane < b && best == low && low < FLT_MAX) & run;
+            const int mid = a + (b - a) / 2;
+            const uint64_t at_hi = at & ~((1ull << mid) - 1ull);
+            int w = mid; // split after position w; boxes without a finite cost: in the middle
+            if (at_hi) w = __builtin_ctzll(at_hi);
+            else if (at) w = 63 - __builtin_clzll(at);
+            axis = (uint32_t)__builtin_amdgcn_ds_bpermute(w << 2, (int)axis);
+            if (at == 0ull) axis = 0u;
+            s_side[axis == 0u ? ord[0] : (axis == 1u ? ord[1] : ord[2])] = on && lane > w ? 1u : 0u;
+            wave_sync();
+            for (int ax = 0; ax < 3; ax++) {
+                const bool side = s_side[ord[ax]] != 0u;
+                const uint64_t right = __ballot(side);
+                const uint32_t p = !on ? (uint32_t)lane
+                                       : (side ? (uint32_t)(w + 1) + (uint32_t)__popcll(right & run & lt)
+                                               : (uint32_t)a + (uint32_t)__popcll(~right & run & lt));
+                s_ord[p] = ord[ax];
+                wave_sync();
+                ord[ax] = s_ord[lane];
+                wave_sync();
             }
-            const uint64_t lmask = __ballot(on && left), rmask = __ballot(on && !left);
-            nl = (uint32_t)__popcll(lmask);
-            const uint64_t below = (1ull << lane) - 1ull;
-            if (!by_bins && mt == 2u) { // two primitives: one each side
-                llo = make_float3(s_box[0][a], s_box[1][a], s_box[2][a]);
-                lhi = make_float3(s_box[3][a], s_box[4][a], s_box[5][a]);
-                rlo = make_float3(s_box[0][b], s_box[1][b], s_box[2][b]);
-                rhi = make_float3(s_box[3][b], s_box[4][b], s_box[5][b]);
-            } else if (!by_bins) { // boxes of the halves
-                const bool il = on && left, ir = on && !left;
-                llo = make_float3(wave_sum_min(blo.x, il), wave_sum_min(blo.y, il), wave_sum_min(blo.z, il));
-                lhi = make_float3(wave_sum_max(bhi.x, il), wave_sum_max(bhi.y, il), wave_sum_max(bhi.z, il));
-                rlo = make_float3(wave_sum_min(blo.x, ir), wave_sum_min(blo.y, ir), wave_sum_min(blo.z, ir));
-                rhi = make_float3(wave_sum_max(bhi.x, ir), wave_sum_max(bhi.y, ir), wave_sum_max(bhi.z, ir));
+            if (on) {
+                if (lane == a) {
+                    const uint32_t g = f + (uint32_t)w;
+                    bt.child[idx] = make_uint2(w == a ? g | kLeafBit : g, w + 1 == b ? (g + 1u) | kLeafBit : g + 1u);
+                    bt.range[idx] = make_uint2(f + (uint32_t)a, f + (uint32_t)b);
+                }
+                slot = 4 * (uint64_t)idx;
+                if (lane <= w) {
+                    b = w;
+                    idx = f + (uint32_t)w;
+                } else {
+                    a = w + 1;
+                    idx = f + (uint32_t)w + 1u;
+                    slot += 2u;
+                }
+                if (a == b) { // a leaf: its box is the primitive's
+                    const uint32_t o = ord[0];
+                    bt.cbox[slot] = make_float4(s_box[0][o], s_box[1][o], s_box[2][o], 0.0f);
+                    bt.cbox[slot + 1] = make_float4(s_box[3][o], s_box[4][o], s_box[5][o], 0.0f);
+                }
             }
-            wave_sync(); // every lane has read the task's positions
-            if (on && mt > 2u) { // move the primitives to their partitioned positions
-                const uint32_t r = a + (left ? (uint32_t)__popcll(lmask & below) : nl + (uint32_t)__popcll(rmask & below));
-                s_box[0][r] = blo.x; s_box[1][r] = blo.y; s_box[2][r] = blo.z;
-                s_box[3][r] = bhi.x; s_box[4][r] = bhi.y; s_box[5][r] = bhi.z;
-                s_cen[0][r] = bc[0]; s_cen[1][r] = bc[1]; s_cen[2][r] = bc[2];
-                s_loc[r] = bloc;
-            }
-            // the node: split after position g; children at g (left) and g + 1 (right)
-            const uint32_t g = a + nl - 1u;
-            const uint32_t lref = nl == 1u ? ((f + a) | kLeafBit) : (f + g);
-            const uint32_t rref = mt - nl == 1u ? ((f + b) | kLeafBit) : (f + g + 1u);
-            if (lane == 0u) {
-                bt.child[idx] = make_uint2(lref, rref);
-                bt.range[idx] = make_uint2(f + a, f + b);
-                float4 *cb = bt.cbox + 4 * (uint64_t)idx;
-                cb[0] = make_float4(llo.x, llo.y, llo.z, 0.0f);
-                cb[1] = make_float4(lhi.x, lhi.y, lhi.z, 0.0f);
-                cb[2] = make_float4(rlo.x, rlo.y, rlo.z, 0.0f);
-                cb[3] = make_float4(rhi.x, rhi.y, rhi.z, 0.0f);
-                if (mt - nl >= 2u) s_task[sp] = make_uint2(((a + nl) << 16) | b, f + g + 1u);
-                if (nl >= 2u) s_task[sp + (mt - nl >= 2u ? 1 : 0)] = make_uint2((a << 16) | g, f + g);
-            }
-            sp += (mt - nl >= 2u ? 1 : 0) + (nl >= 2u ? 1 : 0);
-            wave_sync(); // positions and the task stack written
         }
         // primitives to their final positions
-        if (mine) s_pos[s_loc[lane]] = lane;
+        s_side[ord[0]] = (uint32_t)lane;
         wave_sync();
         if (mine) {
-            const uint32_t pos = f + s_pos[lane];
+            const uint32_t pos = f + s_side[lane];
             ids[pos] = id;
             if (srec) {
                 float4 *dst = reinterpret_cast<float4 *>(srec + pos);
@@ -1118,16 +1090,33 @@ __global__ __launch_bounds__(BLOCK) void k_collapse(LeafBoxes lb, BinaryTree bt,
   }
 }
 
-// Totals of the per-level words (one thread).
-__global__ void k_finish_counts(BuildCounters *ctr) {
+// The end of a build or refit (one wave): totals of the per-level words into the counters, and what the
+// host needs of them into its pinned words. One launch instead of one for the totals and three small
+// device-to-host copies (each about 10 us of the host's and of the stream's time).
+__global__ __launch_bounds__(64) void k_publish_counters(BuildCounters *ctr, const uint32_t *error, HostCounters *host) {
     uint32_t nodes = 0, tris = 0;
-    for (uint32_t l = 0; l < kMaxCollapseLevels; l++) {
+    for (uint32_t l = threadIdx.x; l < kMaxCollapseLevels; l += 64u) {
         const uint64_t w = ctr->level[l];
         nodes += (uint32_t)(w >> 32);
         tris += (uint32_t)w;
     }
+    for (int o = 32; o > 0; o >>= 1) {
+        nodes += (uint32_t)__shfl_xor((int)nodes, o, 64);
+        tris += (uint32_t)__shfl_xor((int)tris, o, 64);
+    }
+    if (threadIdx.x != 0u) return;
     ctr->node_count = nodes;
     ctr->tri_count = tris;
+    host->node_count = nodes;
+    host->tri_count = tris;
+    host->depth = ctr->depth;
+    host->root_ref = ctr->root_ref;
+    for (int k = 0; k < 6; k++) {
+        host->cbounds[k] = ctr->cbounds[k];
+        host->bounds[k] = ctr->bounds[k];
+    }
+    host->tail_level_count = (uint32_t)(ctr->level[kCollapseLaunches] >> 32);
+    host->error = *error;
 }
 
 // Triangle records in leaf order: record i = sorted record order[i]. A node's leaf triangles are
@@ -1480,7 +1469,8 @@ hipError_t bvh_validate(hipStream_t stream, const WideNode *nodes, uint32_t node
 
 // Builds a wide BVH over n primitives (triangles if boxes == nullptr, else boxes).
 // Output arrays: nodes (bvh_node_capacity(n) entries), tris (n entries) or prim_out (n entries).
-// The counters land in `counters_out` (device) for the caller to read back. The build only
+// The counters land in `counters_out` (device), completed and handed to the host by publish_counters;
+// *error_flag is cleared first. The build only
 // enqueues work: every count a step depends on is read on the device, so the host never waits.
 hipError_t bvh_build(hipStream_t stream, void *scratch, size_t scratch_bytes, const void *vbase, uint64_t vstride,
                      uint64_t nverts, const uint32_t *tri, const float4 *boxes, uint32_t n, WideNode *nodes,
@@ -1509,7 +1499,7 @@ hipError_t bvh_build(hipStream_t stream, void *scratch, size_t scratch_bytes, co
     PrimSource src{static_cast<const char *>(vbase), vstride, nverts, tri, boxes, error_flag};
     const uint32_t nslots = n > 1 ? n - 1 : 0;
     hipLaunchKernelGGL(k_init, dim3(std::max<uint32_t>(1, std::min<uint32_t>((nslots + kBlock - 1) / kBlock, 4096))),
-                       dim3(kBlock), 0, stream, ctr, bt.slots, nslots);
+                       dim3(kBlock), 0, stream, ctr, bt.slots, nslots, error_flag);
     if (n == 0) return hipGetLastError();
     const uint32_t grid = (n + kBlock - 1) / kBlock;
     hipLaunchKernelGGL(k_centroid_bounds, dim3(std::min<uint32_t>(grid, 2048)), dim3(kBlock), 0, stream, src, n, ctr);
@@ -1547,7 +1537,7 @@ hipError_t bvh_build(hipStream_t stream, void *scratch, size_t scratch_bytes, co
         const uint32_t phase_grid = (uint32_t)std::max(1, cu_count) * 4u;
         uint64_t estimate = 0;
         if (sah) {
-            // clusters in position order -> ent[0]; each rebuilt by binned SAH, its primitives
+            // clusters in position order -> ent[0]; each rebuilt by sweep SAH, its primitives
             // reordered (ids, and the sorted records of a triangle build)
             const uint32_t nblocks = (n + kPhaseBlock - 1) / kPhaseBlock;
             hipLaunchKernelGGL(k_sah_cut, dim3(nblocks), dim3(kPhaseBlock), 0, stream, n, bt, pend, L.bcount);
@@ -1601,7 +1591,7 @@ hipError_t bvh_build(hipStream_t stream, void *scratch, size_t scratch_bytes, co
     // records are copied from the sorted records in one pass after the last level
     WideOut out{nodes, tris, tris ? pend : prim_out};
     // A root-to-leaf path of the radix tree crosses each of the 30 key bits and 32 index bits at
-    // most once (a binned-SAH cluster adds at most 63 levels below its root), and every wide level
+    // most once (an SAH cluster adds at most 63 levels below its root), and every wide level
     // descends at least one binary level, so the wide depth stays below kCollapseLaunches. The
     // first `head` levels (by default the expected depth, log_width of the primitive count, + 4) are launched over
     // the whole GPU; a launch whose level is empty returns at once. One workgroup then walks any
@@ -1611,24 +1601,32 @@ hipError_t bvh_build(hipStream_t stream, void *scratch, size_t scratch_bytes, co
     for (uint64_t cap = 1; cap < n; cap *= std::max<uint32_t>(width, 2u)) head++;
     if (collapse_head > 0) head = collapse_head; // set by the caller (lc_hip_build_set_collapse_head)
     head = std::min<uint32_t>(head, kCollapseLaunches);
+    uint64_t items = 1; // nodes a level can hold: width^level, and no more than primitives
     for (uint32_t level = 0; level < head; level++) {
+        const uint64_t groups = (items + (uint64_t)cs.block / 8u - 1u) / ((uint64_t)cs.block / 8u);
+        const uint32_t blocks = (uint32_t)std::min<uint64_t>(groups, (uint64_t)grid_collapse);
+        items = std::min<uint64_t>(items * width, n);
         if (cs.block == 1024)
-            hipLaunchKernelGGL((k_collapse<1024, false>), dim3(grid_collapse), dim3(1024), 0, stream, lb, bt, ctr, level,
+            hipLaunchKernelGGL((k_collapse<1024, false>), dim3(blocks), dim3(1024), 0, stream, lb, bt, ctr, level,
                                q0, q1, out, split_small, leaf_max, width);
         else if (cs.block == 512)
-            hipLaunchKernelGGL((k_collapse<512, false>), dim3(grid_collapse), dim3(512), 0, stream, lb, bt, ctr, level,
+            hipLaunchKernelGGL((k_collapse<512, false>), dim3(blocks), dim3(512), 0, stream, lb, bt, ctr, level,
                                q0, q1, out, split_small, leaf_max, width);
         else
-            hipLaunchKernelGGL((k_collapse<256, false>), dim3(grid_collapse), dim3(256), 0, stream, lb, bt, ctr, level,
+            hipLaunchKernelGGL((k_collapse<256, false>), dim3(blocks), dim3(256), 0, stream, lb, bt, ctr, level,
                                q0, q1, out, split_small, leaf_max, width);
     }
     if (head < kCollapseLaunches)
         hipLaunchKernelGGL((k_collapse<512, true>), dim3(1), dim3(512), 0, stream, lb, bt, ctr, head, q0, q1, out,
                            split_small, leaf_max, width);
-    hipLaunchKernelGGL(k_finish_counts, dim3(1), dim3(1), 0, stream, ctr);
     if (tris)
         hipLaunchKernelGGL(k_tri_records, dim3(std::min<uint32_t>(grid, 1u << 20)), dim3(kBlock), 0, stream, pend,
                            (const TriRecord *)srec, tris, n);
+    return hipGetLastError();
+}
+
+hipError_t publish_counters(hipStream_t stream, BuildCounters *ctr, const uint32_t *error, HostCounters *host) {
+    hipLaunchKernelGGL(k_publish_counters, dim3(1), dim3(64), 0, stream, ctr, error, host);
     return hipGetLastError();
 }
 

@@ -51,7 +51,29 @@ __global__ void k_instance_write(InstanceState *st, uint32_t count, uint32_t fie
     }
 }
 
+// The tables of an accel build, read from the pinned staging by one launch: four small copies cost the
+// host and the stream about 10 us each.
+__global__ __launch_bounds__(256) void k_copy_regions(const CopyRegions r) {
+    const uint64_t t = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
+    for (int k = 0; k < 4; k++) {
+        const uint4 *src = static_cast<const uint4 *>(r.src[k]);
+        uint4 *dst = static_cast<uint4 *>(r.dst[k]);
+        for (uint64_t i = t; i < r.bytes[k] / 16u; i += stride) dst[i] = src[i];
+    }
+}
+
 } // namespace
+
+hipError_t copy_regions(hipStream_t stream, const CopyRegions &r) {
+    uint64_t most = 0;
+    for (uint64_t b : r.bytes) {
+        if (b % 16 != 0) return hipErrorInvalidValue;
+        most = std::max(most, b / 16);
+    }
+    if (most == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_copy_regions, dim3((uint32_t)std::min<uint64_t>((most + 255) / 256, 1024)), dim3(256), 0, stream, r);
+    return hipGetLastError();
+}
 
 hipError_t instance_ops(hipStream_t stream, InstanceState *st, uint32_t count, uint32_t field, bool write,
                         const uint32_t *idx, uint32_t n, void *data, uint32_t *err) {

@@ -19,6 +19,17 @@
 namespace lchip {
 
 // ---- kernels (bvh_build.hip) ----
+// What a build or refit leaves for the host, in pinned memory.
+struct HostCounters {
+    uint32_t node_count, tri_count, depth, root_ref;
+    int32_t cbounds[6];
+    float bounds[6];
+    uint32_t tail_level_count; // nodes at wide level kCollapseLaunches: must be 0
+    uint32_t error;
+};
+// Enqueued after a build or refit: its totals into *ctr, and *host (pinned) for the host to read once
+// the stream is past it.
+hipError_t publish_counters(hipStream_t stream, BuildCounters *ctr, const uint32_t *error, HostCounters *host);
 size_t bvh_scratch_bytes(uint32_t n);
 size_t bvh_node_capacity(uint32_t n);
 hipError_t bvh_build(hipStream_t stream, void *scratch, size_t scratch_bytes, const void *vbase, uint64_t vstride,
@@ -48,6 +59,14 @@ hipError_t bvh_validate(hipStream_t stream, const WideNode *nodes, uint32_t node
 // 12 floats per item for transforms, one uint32 otherwise. Indices >= count set *err.
 hipError_t instance_ops(hipStream_t stream, InstanceState *st, uint32_t count, uint32_t field, bool write,
                         const uint32_t *idx, uint32_t n, void *data, uint32_t *err);
+
+// Copies up to 4 regions (16-B aligned, multiples of 16 B) from pinned host memory in one launch.
+struct CopyRegions {
+    const void *src[4];
+    void *dst[4];
+    uint64_t bytes[4];
+};
+hipError_t copy_regions(hipStream_t stream, const CopyRegions &r);
 
 // ---- kernels (trace.hip) ----
 // A batch of rays traced by one launch: rays [start, start + count) of the launch's queue are
@@ -400,14 +419,6 @@ struct Stream {
     bool stop = false;
 };
 
-struct HostCounters {
-    uint32_t node_count, tri_count, depth, root_ref;
-    int32_t cbounds[6];
-    float bounds[6];
-    uint32_t tail_level_count; // nodes at wide level kCollapseLaunches: must be 0
-    uint32_t error;
-};
-
 struct Mesh {
     Device *dev = nullptr;
     std::string name; // DeviceInterface::set_name: build ranges are marked when set
@@ -540,6 +551,6 @@ uint64_t rtc_cache_key(const char *source);
 void rtc_cache_stats(uint64_t *hits, uint64_t *misses);
 // Writes the accel's DeviceAccel descriptor (allocating it on first use) on `stream`, copying
 // from `staging` (pinned, sizeof(DeviceAccel) bytes, untouched until the copy ran).
-int accel_write_descriptor(Accel *a, hipStream_t stream, void *staging);
+int accel_write_descriptor(Accel *a, void *staging); // into the staging; allocates a->desc on first use
 
 } // namespace lchip

@@ -231,13 +231,6 @@ uint32_t leaf_size_for(uint32_t hint) { return hint == LC_HIP_ACCEL_FAST_BUILD ?
 // CPU backend builds Embree's high-quality SAH for FAST_TRACE, cpu/accel.rs:58-62).
 uint32_t sah_for(const Device *dev, uint32_t hint) { return hint != LC_HIP_ACCEL_FAST_BUILD && dev->sah_refine ? 1u : 0u; }
 
-void copy_counters_async(BuildCounters *dctr, HostCounters *host, uint32_t *error, hipStream_t s) {
-    hipMemcpyAsync(host, dctr, offsetof(BuildCounters, level), hipMemcpyDeviceToHost, s);
-    hipMemcpyAsync(&host->tail_level_count, level_nodes_word(dctr, kCollapseLaunches), sizeof(uint32_t),
-                   hipMemcpyDeviceToHost, s);
-    hipMemcpyAsync(&host->error, error, sizeof(uint32_t), hipMemcpyDeviceToHost, s);
-}
-
 // Compacting builds (allow_compaction). cuda_mesh.cpp:42-89 builds into a temporary buffer, reads
 // the compacted size back and copies into the primitive's own buffer, which only grows. Here the
 // tree is built into the device's arena of worst-case wide nodes (n nodes for n primitives) with
@@ -1017,7 +1010,6 @@ int lc_hip_procedural_build(uint64_t device, uint64_t stream, uint64_t primitive
         if (m->allow_compaction) LC_HIP_TRY(arena_acquire(dev, m, n, t));
         StreamScratch *S = stream_scratch(dev, s);
         if (!S) return fail(LC_HIP_ERROR_OUT_OF_MEMORY, "stream scratch");
-        LC_HIP_TRY(hipMemsetAsync(S->error, 0, sizeof(uint32_t), s));
         TimedRegion tr(dev, s, "procedural_build");
         const float *aabb = reinterpret_cast<const float *>(static_cast<const char *>(ab->ptr) + aabb_offset);
         LC_HIP_TRY(aabbs_to_boxes(s, aabb, n, m->proc_boxes));
@@ -1027,7 +1019,7 @@ int lc_hip_procedural_build(uint64_t device, uint64_t stream, uint64_t primitive
                                  S->error, dev->collapse_head);
         if (e != hipSuccess) return hip_fail(e, "procedural bvh_build");
         LC_HIP_TRY(proc_records(s, m->proc_ids, m->proc_boxes, n, m->proc));
-        copy_counters_async(ctr, m->host, S->error, s);
+        LC_HIP_TRY(publish_counters(s, ctr, S->error, m->host));
         if (m->allow_compaction) {
             const int rc = arena_compact(dev, m, s, nullptr);
             if (rc != LC_HIP_OK) return rc;
@@ -1096,7 +1088,7 @@ int lc_hip_mesh_build(uint64_t device, uint64_t stream, uint64_t mesh, uint32_t 
                               m->tris, &ctr, dev->cu_count, S->error);
             }
             if (e != hipSuccess) return hip_fail(e, "bvh_refit");
-            copy_counters_async(ctr, m->host, S->error, s);
+            LC_HIP_TRY(publish_counters(s, ctr, S->error, m->host));
         }
         m->refits++;
         LC_HIP_TRY(hipEventRecord(m->ready, s));
@@ -1125,14 +1117,13 @@ int lc_hip_mesh_build(uint64_t device, uint64_t stream, uint64_t mesh, uint32_t 
         if (m->allow_compaction) LC_HIP_TRY(arena_acquire(dev, m, n, t));
         StreamScratch *S = stream_scratch(dev, s);
         if (!S) return fail(LC_HIP_ERROR_OUT_OF_MEMORY, "stream scratch");
-        LC_HIP_TRY(hipMemsetAsync(S->error, 0, sizeof(uint32_t), s));
         TimedRegion tr(dev, s, "mesh_build");
         BuildCounters *ctr = nullptr;
         hipError_t e = bvh_build(s, t.scratch, t.scratch_bytes, vaddr, vertex_stride, nverts, taddr, nullptr, n,
                                  t.nodes, m->tris, nullptr, &ctr, dev->split_small, leaf_size_for(m->hint),
                                  sah_for(dev, m->hint), dev->bvh_width, dev->cu_count, S->error, dev->collapse_head);
         if (e != hipSuccess) return hip_fail(e, "bvh_build");
-        copy_counters_async(ctr, m->host, S->error, s);
+        LC_HIP_TRY(publish_counters(s, ctr, S->error, m->host));
         if (m->allow_compaction) {
             const int rc = arena_compact(dev, m, s, ctr);
             if (rc != LC_HIP_OK) return rc;
@@ -1388,7 +1379,6 @@ int lc_hip_accel_build(uint64_t device, uint64_t stream, uint64_t accel, uint32_
     a->record_cap = cap / sizeof(InstanceRecord);
     if (instance_count) {
         std::memcpy(a->stage, a->host_records.data(), rec_bytes);
-        LC_HIP_TRY(hipMemcpyAsync(a->records, a->stage, rec_bytes, hipMemcpyHostToDevice, s));
     }
     // the device-side instance table the in-kernel instance ops see (state[count] = error word)
     {
@@ -1404,18 +1394,29 @@ int lc_hip_accel_build(uint64_t device, uint64_t stream, uint64_t accel, uint32_
             st[i].user_id = a->inst[i].user_id;
             st[i].vis_mask = a->inst[i].vis_mask;
         }
-        LC_HIP_TRY(hipMemcpyAsync(a->state, st, state_bytes, hipMemcpyHostToDevice, s));
         a->state_count = instance_count;
         a->state_written = false;
     }
+    // records, instance table, TLAS boxes and descriptor from the staging, in one launch; the staging is
+    // reused by the next build once it ran (no host wait here)
+    const auto upload_tables = [&](size_t boxes) -> int {
+        const int rc = accel_write_descriptor(a, a->stage + off_desc);
+        if (rc != LC_HIP_OK) return rc;
+        static_assert(sizeof(DeviceAccel) % 16 == 0, "copy_regions moves 16 B at a time");
+        const CopyRegions r{{a->stage, a->stage + off_state, a->stage + off_box, a->stage + off_desc},
+                            {a->records, a->state, a->boxes, a->desc},
+                            {rec_bytes, state_bytes, boxes, sizeof(DeviceAccel)}};
+        LC_HIP_TRY(copy_regions(s, r));
+        LC_HIP_TRY(hipEventRecord(a->staged, s));
+        a->stage_pending = true;
+        return LC_HIP_OK;
+    };
     // update_instance_buffer_only (command.h:531-616) refreshes the instance records over the TLAS
     // of the last build; when the instance count differs from that build's (or nothing was built)
     // that TLAS does not describe the instances, so the accel is built in full instead
     if (update_instance_buffer_only && a->built && instance_count == a->tlas_count) {
-        const int rc = accel_write_descriptor(a, s, a->stage + off_desc);
+        const int rc = upload_tables(0);
         if (rc != LC_HIP_OK) return rc;
-        LC_HIP_TRY(hipEventRecord(a->staged, s));
-        a->stage_pending = true;
         return LC_HIP_OK;
     }
     a->built = true;
@@ -1465,7 +1466,6 @@ int lc_hip_accel_build(uint64_t device, uint64_t stream, uint64_t accel, uint32_
         p = a->boxes; cap = a->box_cap;
         LC_HIP_TRY(ensure(p, cap, box_bytes));
         a->boxes = static_cast<float4 *>(p); a->box_cap = cap;
-        LC_HIP_TRY(hipMemcpyAsync(a->boxes, boxes, box_bytes, hipMemcpyHostToDevice, s));
         size_t ncap = bvh_node_capacity(instance_count);
         if (a->tlas_cap < ncap) {
             if (a->tlas_nodes) hipFree(a->tlas_nodes);
@@ -1478,11 +1478,12 @@ int lc_hip_accel_build(uint64_t device, uint64_t stream, uint64_t accel, uint32_
             a->tlas_cap = ncap;
         }
         LC_HIP_TRY(ensure(a->tlas_scratch, a->tlas_scratch_bytes, bvh_scratch_bytes(instance_count)));
+        const int rc = upload_tables(box_bytes);
+        if (rc != LC_HIP_OK) return rc;
         {
             std::lock_guard<std::mutex> dl(dev->mu);
             StreamScratch *S = stream_scratch(dev, s);
             if (!S) return fail(LC_HIP_ERROR_OUT_OF_MEMORY, "stream scratch");
-            LC_HIP_TRY(hipMemsetAsync(S->error, 0, sizeof(uint32_t), s));
             TimedRegion tr(dev, s, "accel_build");
             BuildCounters *ctr = nullptr;
             hipError_t e = bvh_build(s, a->tlas_scratch, a->tlas_scratch_bytes, nullptr, 0, 0, nullptr, a->boxes,
@@ -1491,18 +1492,14 @@ int lc_hip_accel_build(uint64_t device, uint64_t stream, uint64_t accel, uint32_
                                      std::max(1, dev->cu_count),
                                      S->error, dev->collapse_head);
             if (e != hipSuccess) return hip_fail(e, "tlas build");
-            copy_counters_async(ctr, a->tlas_host, S->error, s);
+            LC_HIP_TRY(publish_counters(s, ctr, S->error, a->tlas_host));
         }
         LC_HIP_TRY(hipEventRecord(a->tlas_ready, s));
         a->tlas_valid = true;
-    }
-    {
-        const int rc = accel_write_descriptor(a, s, a->stage + off_desc);
+    } else {
+        const int rc = upload_tables(0);
         if (rc != LC_HIP_OK) return rc;
     }
-    // the staging is reused by the next build once these copies ran (no host wait here)
-    LC_HIP_TRY(hipEventRecord(a->staged, s));
-    a->stage_pending = true;
     return LC_HIP_OK;
 }
 
@@ -1510,7 +1507,7 @@ int lc_hip_accel_build(uint64_t device, uint64_t stream, uint64_t accel, uint32_
 
 // The DeviceAccel descriptor of lc_hip_device.h: the query view of the accel (as
 // lc_hip_accel_query builds it) plus the instance table.
-int lchip::accel_write_descriptor(Accel *a, hipStream_t s, void *staging) {
+int lchip::accel_write_descriptor(Accel *a, void *staging) {
     DeviceAccel &d = a->desc_host;
     std::memset(&d, 0, sizeof(d));
     const uint32_t n = (uint32_t)a->inst.size();
@@ -1530,7 +1527,6 @@ int lchip::accel_write_descriptor(Accel *a, hipStream_t s, void *staging) {
     d.error = a->dev->error;
     if (!a->desc) LC_HIP_TRY(hipMalloc(&a->desc, sizeof(DeviceAccel)));
     std::memcpy(staging, &d, sizeof(d));
-    LC_HIP_TRY(hipMemcpyAsync(a->desc, staging, sizeof(d), hipMemcpyHostToDevice, s));
     return LC_HIP_OK;
 }
 
