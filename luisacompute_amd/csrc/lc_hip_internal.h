@@ -266,10 +266,13 @@ struct QueryParams {
     const float4 *rays; // 2 float4 per ray
     void *hits;         // 24-B CommittedHit per ray
     const uint32_t *order; // optional: queue slot -> ray (sorted queue), else identity
-    uint32_t *counter;  // queue slot counter (zeroed by the launch)
+    uint32_t *ray_counter; // queue slot counters (zeroed by the launch)
     uint32_t count;
     uint32_t mask;
     uint32_t first;     // terminate on the first commit (traverse_any)
+    // nearest-commit queries: as in TraceParams
+    int steps;
+    uint32_t fetch_chunk, fetch_segments, tri_quarters, refill_below, lanes;
     QueryGeometry geo;
     uint2 *spill;
     uint32_t spill_depth;
@@ -278,9 +281,9 @@ struct QueryParams {
     float cutout;
     uint32_t procedural_mode;
 };
-int query_block();
+int query_block(bool first);
 int query_lds_entries();
-int query_blocks_per_cu();
+int query_blocks_per_cu(bool first);
 hipError_t query_launch(const QueryParams &P, hipStream_t stream, int grid);
 
 bool trace_config_supported(int block, int slds);

@@ -20,6 +20,7 @@
 
 #include "lc_hip_internal.h"
 #include "ray_query.h"
+#include "wave_walker.h"
 
 namespace lchip {
 
@@ -58,13 +59,51 @@ struct BuiltinPolicy {
     }
 };
 
+// Nearest-commit queries as the other mode of WaveWalker: the wave's lanes share the callbacks' work as
+// they share plain triangle tests. (An answer is the minimum over the committed candidates, and the
+// callbacks are functions of the candidate alone.)
+struct QueryMode {
+    using Params = QueryParams;
+    static constexpr bool kQuery = true;
+    static constexpr uint32_t kMiss = rq::kHitMiss, kSurface = rq::kHitSurface, kProcedural = rq::kHitProcedural;
+    __device__ __forceinline__ static void locate(const Params &, uint32_t q, uint32_t &batch, uint32_t &ray) {
+        batch = 0u;
+        ray = q;
+    }
+    __device__ __forceinline__ static const float4 *rays(const Params &P, uint32_t) { return P.rays; }
+    __device__ __forceinline__ static uint32_t mask(const Params &P, uint32_t) { return P.mask; }
+    __device__ __forceinline__ static char *out(const Params &P, uint32_t) { return static_cast<char *>(P.hits); }
+    __device__ __forceinline__ static bool surface(const Params &P, uint32_t inst, uint32_t prim, float u, float v, float t) {
+        return BuiltinPolicy{P.surface_mode, P.cutout, P.procedural_mode}.surface(inst, prim, u, v, t);
+    }
+    __device__ __forceinline__ static bool procedural(const Params &P, uint32_t inst, uint32_t prim, const float o[3],
+                                                      const float d[3], float4 lo, float4 hi, float &t) {
+        return BuiltinPolicy{P.surface_mode, P.cutout, P.procedural_mode}.procedural(inst, prim, o, d, nullptr, nullptr,
+                                                                                     lo, hi, 0.0f, t);
+    }
+};
+
+constexpr int kNearestBlock = 64;
+
+// One wave per workgroup: its LDS (6,400 B) and registers let 5 run on each SIMD. 2.1M queries over
+// 524,288 cutout triangles and as many spheres 4,905 -> 3,608 us, 5,000 queries over 1,000 of each
+// 1,207 -> 227 us (one query per lane, wave-uniform leaf and node steps, before).
+__global__ __launch_bounds__(kNearestBlock) __attribute__((amdgpu_waves_per_eu(5)))
+void k_query_nearest(const QueryParams P) {
+    __shared__ trav::WaveShared<false, kNearestBlock, 8> shared;
+    trav::WaveWalker<false, true, false, kNearestBlock, 8, QueryMode> W;
+    W.init(P, &shared, threadIdx.x);
+    W.trace_queue(P, P.count);
+}
+
+// First-commit queries (traverse_any): one query per lane, each lane stopping at its first commit.
 constexpr int kQueryBlock = 128;
 constexpr int kQuerySlds = 8;
 constexpr int kQuerySteps = 16;     // walk steps between refills of finished lanes
 constexpr uint32_t kQueryChunk = 256; // queue slots a wave claims per atomic
 
 __global__ void k_query_zero(uint32_t *counter) {
-    if (threadIdx.x == 0) *counter = 0u;
+    if (threadIdx.x < kFetchSegments) counter[threadIdx.x * kCounterStride] = 0u;
 }
 
 // Persistent launch: a wave claims kQueryChunk queue slots per atomic and hands them to its idle
@@ -98,7 +137,7 @@ __global__ __launch_bounds__(kQueryBlock) void k_query(const QueryParams P) {
             } else {
                 const uint32_t leader = (uint32_t)__ffsll((long long)need) - 1u;
                 uint32_t b = 0;
-                if (lane == leader) b = atomicAdd(P.counter, kQueryChunk);
+                if (lane == leader) b = atomicAdd(P.ray_counter, kQueryChunk);
                 b = __builtin_amdgcn_readlane(b, (int)leader);
                 const uint32_t nb = min(b, count), ne = (uint32_t)min<uint64_t>((uint64_t)b + kQueryChunk, count);
                 drained = (uint64_t)b + kQueryChunk >= count;
@@ -130,19 +169,22 @@ __global__ __launch_bounds__(kQueryBlock) void k_query(const QueryParams P) {
 
 } // namespace
 
-int query_block() { return kQueryBlock; }
+int query_block(bool first) { return first ? kQueryBlock : kNearestBlock; }
 int query_lds_entries() { return kQuerySlds; }
 
-int query_blocks_per_cu() {
+int query_blocks_per_cu(bool first) {
     int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_query, kQueryBlock, 0) != hipSuccess || n < 1) n = 1;
-    return n;
+    const hipError_t e = first ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_query, kQueryBlock, 0)
+                               : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_query_nearest, kNearestBlock, 0);
+    return e == hipSuccess && n > 0 ? n : 1;
 }
 
 hipError_t query_launch(const QueryParams &P, hipStream_t stream, int grid) {
     if (P.count == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_query_zero, dim3(1), dim3(64), 0, stream, P.counter);
-    hipLaunchKernelGGL(k_query, dim3(grid), dim3(kQueryBlock), 0, stream, P);
+    if (P.first != 0u || P.lanes == 0u)
+        hipLaunchKernelGGL(k_query_zero, dim3(1), dim3(64), 0, stream, P.ray_counter);
+    if (P.first != 0u) hipLaunchKernelGGL(k_query, dim3(grid), dim3(kQueryBlock), 0, stream, P);
+    else hipLaunchKernelGGL(k_query_nearest, dim3(grid), dim3(kNearestBlock), 0, stream, P);
     return hipGetLastError();
 }
 

@@ -2020,10 +2020,23 @@ int lc_hip_accel_query(uint64_t device, uint64_t stream, uint64_t accel, uint64_
     P.cutout = policy->cutout;
     P.procedural_mode = policy->procedural_mode;
     std::lock_guard<std::mutex> dl(dev->mu);
-    const int block = query_block();
-    const uint64_t want = ((uint64_t)ray_count + block - 1) / block;
-    const int grid = (int)std::max<uint64_t>(
-        1, std::min<uint64_t>((uint64_t)query_blocks_per_cu() * std::max(1, dev->cu_count), want));
+    const bool first = P.first != 0u;
+    const TraceConfig &cfg = dev->cfg[first ? 1 : 0];
+    const int block = query_block(first), bpc = query_blocks_per_cu(first), cus = std::max(1, dev->cu_count);
+    int grid;
+    if (first) {
+        const uint64_t want = ((uint64_t)ray_count + block - 1) / block;
+        grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)bpc * cus, want));
+    } else {
+        const TraceGrid tg = trace_grid(ray_count, block, bpc, cus);
+        grid = tg.grid;
+        P.lanes = tg.lanes;
+    }
+    P.steps = cfg.steps;
+    P.fetch_chunk = cfg.fetch_chunk;
+    P.fetch_segments = cfg.fetch_segments;
+    P.tri_quarters = cfg.tri_quarters;
+    P.refill_below = cfg.refill_below;
     const uint32_t slds = (uint32_t)query_lds_entries();
     P.spill_depth = stack_need > slds ? stack_need - slds : 0u;
     StreamScratch *S = stream_scratch(dev, s);
@@ -2031,10 +2044,10 @@ int lc_hip_accel_query(uint64_t device, uint64_t stream, uint64_t accel, uint64_
     LC_HIP_GROW((S, s, S->spill, S->spill_bytes, (size_t)grid * block * P.spill_depth * sizeof(uint2)));
     P.spill = static_cast<uint2 *>(S->spill);
     P.error = S->error;
-    P.counter = S->ray_counter;
+    P.ray_counter = S->ray_counter;
     // the query queue is sorted like trace queues when ray sorting is on (per-ray answers of the
     // nearest-commit query do not depend on the order); under capture as for traces
-    bool sort = dev->cfg[P.first ? 1 : 0].sort_rays && ray_count > 1 && !P.geo.empty;
+    bool sort = cfg.sort_rays && ray_count >= kSortMinRays && !P.geo.empty && (!P.geo.two || a->box_overlap >= kSortMinOverlap);
     if (sort && capturing(s) && S->sort_bytes < ray_sort_scratch_bytes(ray_count)) sort = false;
     if (sort) LC_HIP_GROW((S, s, S->sort, S->sort_bytes, ray_sort_scratch_bytes(ray_count)));
     TimedRegion tr(dev, s, P.first ? "query_any" : "query");

@@ -64,109 +64,12 @@ template<bool ANY, bool TWO, bool COUNT, int BLOCK, int SLDS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(SLDS == 8 ? (TWO ? 5 : 6) : 1)))
 void k_trace(const TraceParams P) {
     __shared__ trav::WaveShared<ANY, BLOCK, SLDS> shared;
-    const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t count = P.count_ptr ? min(*P.count_ptr, P.count) : P.count;
     trav::WaveWalker<ANY, TWO, COUNT, BLOCK, SLDS> W;
     W.init(P, &shared, tid);
 
-    // Fetching: the queue is split into kFetchSegments contiguous segments, one per XCD
-    // (workgroups are dealt to the XCDs round-robin, so block b runs on XCD b mod 8), each with a
-    // slot counter on its own cache line. A wave claims `chunk` slots of its segment per atomic
-    // and hands them to its idle lanes from that pool; when the segment is used up it takes
-    // slots from the others. One counter address serialises its atomics (about 85M/s), so a
-    // per-round atomic on one counter would cap the launch; a segment per XCD also keeps each
-    // XCD's L2 on one region of a sorted queue.
-    // fetch_chunk 0 claims exactly the slots the idle lanes need (the narrowest window of the
-    // queue in flight, one atomic per refill round); fetch_segments 1 or kFetchSegments.
-    const uint32_t waves = gridDim.x * (BLOCK / 64);
-    const uint32_t chunk = P.fetch_chunk ? max(64u, min(P.fetch_chunk, (count / max(1u, waves * 4u)) & ~63u)) : 0u;
-    const uint32_t nseg = P.fetch_segments > 1 ? kFetchSegments : 1u;
-    const uint32_t seg0 = blockIdx.x % nseg;
-    const bool simple = chunk == 0u && nseg == 1u;
-    uint32_t pool = 0, pool_end = 0; // wave-uniform: unclaimed slots [pool, pool_end)
-    bool drained = false;            // wave-uniform: every segment is used up
-    bool active = false, exhausted = false;
-    if (P.lanes != 0u) {
-        // every ray has a lane: wave w takes the slots [w lanes, w lanes + lanes) of the queue, with
-        // w counted XCD by XCD (block b runs on XCD b mod 8), so that each XCD has its own part
-        const uint32_t per_xcd = gridDim.x / kFetchSegments;
-        const uint32_t b = (blockIdx.x % kFetchSegments) * per_xcd + blockIdx.x / kFetchSegments;
-        const uint64_t w = (uint64_t)b * (BLOCK / 64) + (tid >> 6);
-        const uint64_t my = w * P.lanes + lane;
-        drained = exhausted = true;
-        if (lane < P.lanes && my < count) {
-            const uint32_t q = P.order ? P.order[my] : (uint32_t)my;
-            const uint32_t bt = find_batch(P.batches, q);
-            W.start(P, bt, q - P.batches.b[bt].start);
-            active = true;
-        }
-    }
-    uint64_t rounds = 0; // counting form: refill rounds of this wave
-    for (;;) {
-        const uint64_t need = __ballot(!active && !exhausted);
-        if (need) {
-            const uint32_t n_need = (uint32_t)__popcll(need);
-            const uint32_t rank = (uint32_t)__popcll(need & ((1ull << lane) - 1ull));
-            const uint32_t avail = pool_end - pool;
-            uint32_t my = rank < avail ? pool + rank : 0xFFFFFFFFu; // lanes served by the pool
-            if (simple) {
-                // one counter, exactly the slots the idle lanes need
-                const uint32_t leader = (uint32_t)__ffsll((long long)need) - 1u;
-                uint32_t b = 0;
-                if (lane == leader) b = atomicAdd(P.ray_counter, n_need);
-                b = __builtin_amdgcn_readlane(b, (int)leader);
-                my = b + rank;
-                drained = b + n_need >= count;
-            } else if (avail >= n_need) {
-                pool += n_need;
-            } else if (drained) {
-                pool = pool_end;
-            } else {
-                // refill: the leader claims a chunk of this XCD's segment, else of another one
-                const uint32_t leader = (uint32_t)__ffsll((long long)need) - 1u;
-                uint32_t nb = 0, ne = 0;
-                if (lane == leader) {
-                    const uint32_t claim = chunk ? chunk : n_need - avail;
-                    for (uint32_t k = 0; k < nseg; k++) {
-                        const uint32_t s = (seg0 + k) % nseg;
-                        const uint32_t lo = (uint32_t)((uint64_t)count * s / nseg);
-                        const uint32_t hi = (uint32_t)((uint64_t)count * (s + 1) / nseg);
-                        if (lo == hi) continue;
-                        const uint32_t b = atomicAdd(P.ray_counter + s * kCounterStride, claim);
-                        if (b < hi - lo) {
-                            nb = lo + b;
-                            ne = lo + min(b + claim, hi - lo);
-                            break;
-                        }
-                    }
-                }
-                nb = __builtin_amdgcn_readlane(nb, (int)leader); // wave-uniform from here on
-                ne = __builtin_amdgcn_readlane(ne, (int)leader);
-                drained = nb == ne;
-                if (rank >= avail && rank - avail < ne - nb) my = nb + (rank - avail);
-                pool = nb + min(n_need - avail, ne - nb);
-                pool_end = ne;
-            }
-            if (!active && !exhausted) {
-                if (my < count) {
-                    const uint32_t q = P.order ? P.order[my] : my; // sorted queue: fetch in key order
-                    const uint32_t b = find_batch(P.batches, q);
-                    W.start(P, b, q - P.batches.b[b].start);
-                    active = true;
-                } else if (drained) {
-                    exhausted = true; // no slot left in any segment (else: retry next round)
-                }
-            }
-        }
-        if (!__any(active)) break;
-        if (COUNT && lane == (uint32_t)__ffsll((long long)__ballot(1)) - 1u) rounds++;
-        W.run(P, active, !drained);
-        if (active && W.finished()) {
-            if (!COUNT) W.write(P); // the counting form has no output buffers (out is null)
-            active = false;
-        }
-    }
+    const uint64_t rounds = W.trace_queue(P, count); // counting form: refill rounds of this wave
     if (COUNT) {
         // stats: node visits, triangle tests, live lane-iterations, wave iterations, refill rounds
         uint64_t v[5] = {W.n_nodes, W.n_tris, W.n_live, W.n_wave, rounds};

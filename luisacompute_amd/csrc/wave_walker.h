@@ -69,9 +69,26 @@ struct WaveShared {
     uint32_t rec[ANY ? 1 : BLOCK];
 };
 
-template<bool ANY, bool TWO, bool COUNT, int BLOCK, int SLDS>
+// What is traced and where its rays and results are: plain traces over ray batches. (query.hip has the
+// other mode: nearest-commit ray queries, whose candidates go through callbacks.)
+struct TraceMode {
+    using Params = TraceParams;
+    static constexpr bool kQuery = false;
+    __device__ __forceinline__ static void locate(const Params &P, uint32_t q, uint32_t &batch, uint32_t &ray) {
+        batch = find_batch(P.batches, q);
+        ray = q - P.batches.b[batch].start;
+    }
+    __device__ __forceinline__ static const float4 *rays(const Params &P, uint32_t batch) { return P.batches.b[batch].rays; }
+    __device__ __forceinline__ static uint32_t mask(const Params &P, uint32_t batch) { return P.batches.b[batch].mask; }
+    __device__ __forceinline__ static char *out(const Params &P, uint32_t batch) { return static_cast<char *>(P.batches.b[batch].out); }
+};
+
+template<bool ANY, bool TWO, bool COUNT, int BLOCK, int SLDS, class Mode = TraceMode>
 struct WaveWalker {
     using Shared = WaveShared<ANY, BLOCK, SLDS>;
+    using Params = typename Mode::Params;
+    static constexpr bool kQuery = Mode::kQuery;
+    static_assert(!kQuery || (TWO && !ANY && !COUNT), "queries: nearest commit over instances");
     Shared *sh;
     uint2 *queue;          // this wave's queue
     uint32_t tid, lane;
@@ -86,6 +103,7 @@ struct WaveWalker {
     uint32_t g_base, g_mask, t_base, t_mask;
     int floor;             // stack height of the current level: 0, or where the instance was entered
     uint32_t cur_inst;     // instance this lane is in (two-level; kWorld: in the TLAS)
+    uint32_t cur_flags;    // queries: its InstanceRecord flags
     const WideNode *nodes;
     const TriRecord *tris;
     uint64_t n_nodes, n_tris, n_live, n_wave; // counting form only, as in Walker
@@ -93,29 +111,36 @@ struct WaveWalker {
     static constexpr uint32_t kWorld = 0xFFFFFFFFu;
     __device__ __forceinline__ bool in_blas() const { return !TWO || cur_inst != kWorld; }
 
-    __device__ __forceinline__ void init(const TraceParams &P, Shared *shared, uint32_t t) {
+    __device__ __forceinline__ void init(const Params &P, Shared *shared, uint32_t t) {
         sh = shared; tid = t; lane = t & 63u; queue = shared->queue[t >> 6];
         head = tail = last = 0u;
         sp = floor = 0; g_mask = t_mask = 0u; any_hit = false;
         n_nodes = 0; n_tris = 0; n_live = 0; n_wave = 0;
-        nodes = TWO ? P.geo.tlas_nodes : P.geo.blas_nodes;
-        tris = P.geo.blas_tris;
-        cur_inst = TWO ? kWorld : 0u;
+        if constexpr (TWO) {
+            nodes = P.geo.tlas_nodes;
+            tris = nullptr;
+            cur_inst = kWorld;
+        } else {
+            nodes = P.geo.blas_nodes;
+            tris = P.geo.blas_tris;
+            cur_inst = 0u;
+        }
+        cur_flags = 0u;
         batch = ray = 0u;
     }
 
     // This lane's spill entry k. As in Walker the host sizes spill_depth from the built depths; the
     // checks only guard memory.
-    __device__ __forceinline__ uint2 *spill_at(const TraceParams &P, int k) const {
+    __device__ __forceinline__ uint2 *spill_at(const Params &P, int k) const {
         return P.spill + ((uint64_t)blockIdx.x * BLOCK + tid) * P.spill_depth + k;
     }
-    __device__ __forceinline__ void push(const TraceParams &P, uint2 e) {
+    __device__ __forceinline__ void push(const Params &P, uint2 e) {
         if (sp < SLDS) sh->stk[sp][tid] = e;
         else if ((uint32_t)(sp - SLDS) < P.spill_depth) *spill_at(P, sp - SLDS) = e;
         else atomicOr(P.error, 1u);
         sp++;
     }
-    __device__ __forceinline__ uint2 pop(const TraceParams &P) {
+    __device__ __forceinline__ uint2 pop(const Params &P) {
         sp--;
         if (sp < SLDS) return sh->stk[sp][tid];
         if ((uint32_t)(sp - SLDS) < P.spill_depth) return *spill_at(P, sp - SLDS);
@@ -127,19 +152,19 @@ struct WaveWalker {
     }
 
     // Ray `r` of batch `b` as the launch was given it.
-    __device__ __forceinline__ void load_ray(const TraceParams &P, float o[3], float d[3], float &lo, float &hi) const {
-        const float4 *rays = P.batches.b[batch].rays;
+    __device__ __forceinline__ void load_ray(const Params &P, float o[3], float d[3], float &lo, float &hi) const {
+        const float4 *rays = Mode::rays(P, batch);
         const float4 r0 = rays[2 * (uint64_t)ray], r1 = rays[2 * (uint64_t)ray + 1];
         o[0] = r0.x; o[1] = r0.y; o[2] = r0.z; lo = r0.w;
         d[0] = r1.x; d[1] = r1.y; d[2] = r1.z; hi = r1.w;
     }
-    __device__ __forceinline__ uint2 *out_hit(const TraceParams &P) const {
-        return reinterpret_cast<uint2 *>(static_cast<char *>(P.batches.b[batch].out) + 24ull * ray);
+    __device__ __forceinline__ uint2 *out_hit(const Params &P) const {
+        return reinterpret_cast<uint2 *>(Mode::out(P, batch) + 24ull * ray);
     }
 
     // A new ray for this lane (called by the lanes that take one).
-    __device__ __forceinline__ void start(const TraceParams &P, uint32_t b, uint32_t r) {
-        const Geometry &G = P.geo;
+    __device__ __forceinline__ void start(const Params &P, uint32_t b, uint32_t r) {
+        const auto &G = P.geo;
         batch = b;
         ray = r;
         t_best = FLT_MAX * 2.0f; // +inf
@@ -151,17 +176,24 @@ struct WaveWalker {
         float o[3], d[3];
         load_ray(P, o, d, tmin, tmax);
         reset_key(t_best);
-        if (TWO) {
+        if constexpr (TWO) {
             for (int k = 0; k < 3; k++) { R.o[k] = o[k]; R.d[k] = d[k]; }
             cur_inst = kWorld;
             nodes = G.tlas_nodes;
             ray_setup(R);
             g_mask = G.empty ? 0u : ((1u << R.oct) | (1u << 8));
+            if constexpr (kQuery) {
+                if (!G.two) { // one instance and no TLAS: instance 0 is entered next
+                    g_mask = 0u;
+                    t_base = 0u;
+                    t_mask = G.empty ? 0u : 1u;
+                }
+            }
         } else {
             xform_point(G.inst_inv, o, R.o);
             xform_vector(G.inst_inv, d, R.d);
             ray_setup(R);
-            g_mask = (G.empty || (G.inst_mask & P.batches.b[b].mask & 0xFFu) == 0u) ? 0u : ((1u << R.oct) | (1u << 8));
+            g_mask = (G.empty || (G.inst_mask & Mode::mask(P, b) & 0xFFu) == 0u) ? 0u : ((1u << R.oct) | (1u << 8));
         }
     }
 
@@ -198,7 +230,7 @@ struct WaveWalker {
     }
 
     // Tests up to 64 pairs of the queue, one per lane.
-    __device__ __forceinline__ void triangle_step() {
+    __device__ __forceinline__ void triangle_step(const Params &P) {
         const uint32_t n = min(64u, tail - head);
         const bool on = lane < n;
         const uint2 e = queue[(head + lane) & (kTriQueue - 1u)];
@@ -216,8 +248,27 @@ struct WaveWalker {
         }
         bool hit = false;
         float t = 0.0f, u = 0.0f, v = 0.0f;
-        uint32_t prim = 0u;
-        if (on) {
+        uint32_t prim = 0u, procedural = 0u;
+        if constexpr (kQuery) {
+            const uint32_t inst = from_lane(from, cur_inst), flags = from_lane(from, cur_flags);
+            procedural = on && (flags & kInstProcedural) ? 1u : 0u;
+            if (__ballot(procedural != 0u) != 0ull) { // the callback takes the object-space ray
+                r.d[0] = from_lane(from, R.d[0]); r.d[1] = from_lane(from, R.d[1]); r.d[2] = from_lane(from, R.d[2]);
+                if (procedural) {
+                    const float4 *pr = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(base) + 32ull * e.x);
+                    const float4 b0 = pr[0], b1 = pr[1];
+                    prim = __float_as_uint(b0.w);
+                    hit = Mode::procedural(P, inst, prim, r.o, r.d, b0, b1, t) && t >= lo && t < hi;
+                }
+            }
+            if (on && !procedural) {
+                const float4 *tr = reinterpret_cast<const float4 *>(base + e.x);
+                const float4 a = tr[0], b = tr[1], c = tr[2];
+                prim = __float_as_uint(a.w);
+                hit = wt_intersect(r, a, b, c, lo, hi, t, u, v) &&
+                      ((flags & kInstOpaque) || Mode::surface(P, inst, prim, u, v, t));
+            }
+        } else if (on) {
             const float4 *tr = reinterpret_cast<const float4 *>(base + e.x);
             const float4 a = tr[0], b = tr[1], c = tr[2];
             if (COUNT) n_tris++;
@@ -249,7 +300,7 @@ struct WaveWalker {
                 const uint32_t w = (tid & ~63u) + owner;
                 sh->u[w] = u;
                 sh->v[w] = v;
-                sh->rec[w] = e.x | (__float_as_uint(t) == 0x80000000u ? kNegZero : 0u);
+                sh->rec[w] = (kQuery ? procedural : e.x) | (__float_as_uint(t) == 0x80000000u ? kNegZero : 0u);
             }
             lds_order();
             t_best = t_value((uint32_t)(sh->key[tid] >> 32));
@@ -257,8 +308,8 @@ struct WaveWalker {
     }
 
     // Leaves the current instance and / or enters the next one (called by the lanes with inst_work()).
-    __device__ __forceinline__ void instance_step(const TraceParams &P) {
-        const Geometry &G = P.geo;
+    __device__ __forceinline__ void instance_step(const Params &P) {
+        const auto &G = P.geo;
         float o[3], d[3], lo, hi;
         load_ray(P, o, d, lo, hi);
         bool world = false; // the world-space ray is needed again
@@ -276,7 +327,7 @@ struct WaveWalker {
                         if (any_hit) {
                             const uint2 *h = out_hit(P);
                             const uint2 h0 = h[0];
-                            better = nearer(t, cur_inst, prim, __uint_as_float(h[2].x), h0.x, h0.y);
+                            better = nearer(t, cur_inst, prim, __uint_as_float(kQuery ? h[2].y : h[2].x), h0.x, h0.y);
                         }
                         if (better) store_hit(P, k, cur_inst);
                         any_hit = true;
@@ -301,13 +352,17 @@ struct WaveWalker {
         while (t_mask != 0u) {
             const uint32_t b = (uint32_t)__builtin_ctz(t_mask);
             t_mask &= t_mask - 1u;
-            const uint32_t id = G.tlas_prims[t_base + b];
+            uint32_t id = 0u;
+            if constexpr (kQuery) id = G.two ? G.tlas_prims[t_base + b] : 0u;
+            else id = G.tlas_prims[t_base + b];
             const InstanceRecord *ir = G.instances + id;
             const uint32_t imask = ir->vis_mask;
             const uint64_t bn = ir->blas_nodes;
             // procedural primitives report only to ray queries (plain traces run without
             // intersection functions, cpu/accel.rs:476-484)
-            if (bn == 0u || (imask & P.batches.b[batch].mask & 0xFFu) == 0u || (ir->flags & kInstProcedural)) continue;
+            const uint32_t iflags = ir->flags;
+            if (bn == 0u || (imask & Mode::mask(P, batch) & 0xFFu) == 0u || (!kQuery && (iflags & kInstProcedural))) continue;
+            cur_flags = iflags;
             if ((g_mask & 0xFFu) != 0u) push(P, make_uint2(g_base, g_mask));
             if (t_mask != 0u) push(P, make_uint2(t_base, t_mask | kInstGroup));
             t_mask = 0u;
@@ -337,7 +392,7 @@ struct WaveWalker {
     }
 
     // Visits the next node of this lane (called by the lanes with node_work()).
-    __device__ __forceinline__ void visit(const TraceParams &P) {
+    __device__ __forceinline__ void visit(const Params &P) {
         if ((g_mask & 0xFFu) == 0u) {
             const uint2 e = pop(P);
             if (TWO && (e.y & kInstGroup)) {
@@ -388,7 +443,7 @@ struct WaveWalker {
     // (1080p room: 16.5 ms with fixed quarters for both kinds, 15.5 so; 1M soup 1,246 -> 1,209 us.)
     // Returns when no lane has work left, or, with P.refill_below > 0 and rays to hand out
     // (can_refill), once fewer lanes than that are busy.
-    __device__ __forceinline__ void run(const TraceParams &P, bool active, bool can_refill) {
+    __device__ __forceinline__ void run(const Params &P, bool active, bool can_refill) {
         const uint32_t full = 16u * (P.tri_quarters ? P.tri_quarters : (uint32_t)kTriQuarters);
         const uint32_t refill_below = can_refill ? P.refill_below : 0u;
         for (int it = 0; it < P.steps; it++) {
@@ -412,7 +467,7 @@ struct WaveWalker {
                 tri = true;
             }
             if (COUNT) account((active && !finished()) || (tri && lane < queued));
-            if (tri) triangle_step();
+            if (tri) triangle_step(P);
             else if (work) visit(P);
             queue_triangles(active);
         }
@@ -421,27 +476,127 @@ struct WaveWalker {
     static constexpr unsigned long long kMissKey = 0xFFFFFFFFull;
     // Writes the ray's closest-hit record (24-B SurfaceHit) for the nearest hit `k` of instance `inst`;
     // the padding word carries the leaf record with P.hit_record (queues of the path tracer).
-    __device__ __forceinline__ void store_hit(const TraceParams &P, unsigned long long k, uint32_t inst) const {
+    __device__ __forceinline__ void store_hit(const Params &P, unsigned long long k, uint32_t inst) const {
         uint2 *h = out_hit(P);
         const uint32_t prim = (uint32_t)k;
-        if (prim == 0xFFFFFFFFu) {
-            h[0] = make_uint2(0xFFFFFFFFu, 0xFFFFFFFFu);
-            h[1] = make_uint2(0u, 0u);
-            h[2] = make_uint2(__float_as_uint(tmax), 0u);
-        } else {
-            const uint32_t rec = sh->rec[tid];
-            h[0] = make_uint2(inst, prim);
-            h[1] = make_uint2(__float_as_uint(sh->u[tid]), __float_as_uint(sh->v[tid]));
-            h[2] = make_uint2((rec & kNegZero) ? kNegZero : __float_as_uint(t_value((uint32_t)(k >> 32))),
-                              P.hit_record ? (rec & ~kNegZero) : 0u);
-        }
+        const bool hit = prim != 0xFFFFFFFFu;
+        const uint32_t rec = hit ? sh->rec[tid] : 0u;
+        const uint32_t t = !hit ? __float_as_uint(tmax)
+                                : ((rec & kNegZero) ? kNegZero : __float_as_uint(t_value((uint32_t)(k >> 32))));
+        h[0] = make_uint2(hit ? inst : 0xFFFFFFFFu, prim);
+        h[1] = hit ? make_uint2(__float_as_uint(sh->u[tid]), __float_as_uint(sh->v[tid])) : make_uint2(0u, 0u);
+        if constexpr (kQuery) h[2] = make_uint2(!hit ? Mode::kMiss : ((rec & 1u) ? Mode::kProcedural : Mode::kSurface), t);
+        else h[2] = make_uint2(t, hit && P.hit_record ? (rec & ~kNegZero) : 0u);
     }
 
     // The result of a finished ray (two-level closest hits were written as instances were left).
-    __device__ __forceinline__ void write(const TraceParams &P) const {
-        if (ANY) static_cast<uint8_t *>(P.batches.b[batch].out)[ray] = any_hit ? 1u : 0u;
+    __device__ __forceinline__ void write(const Params &P) const {
+        if (ANY) reinterpret_cast<uint8_t *>(Mode::out(P, batch))[ray] = any_hit ? 1u : 0u;
         else if (!TWO) store_hit(P, sh->key[tid], 0u);
         else if (!any_hit) store_hit(P, kMissKey, 0u);
+    }
+
+    // Traces the first `count` rays of the launch's queue with this wave and the launch's others;
+    // returns the rounds of handing out rays.
+    __device__ __forceinline__ uint64_t trace_queue(const Params &P, uint32_t count) {
+        uint64_t rounds = 0;
+        // Fetching: the queue is split into kFetchSegments contiguous segments, one per XCD
+        // (workgroups are dealt to the XCDs round-robin, so block b runs on XCD b mod 8), each with a
+        // slot counter on its own cache line. A wave claims `chunk` slots of its segment per atomic
+        // and hands them to its idle lanes from that pool; when the segment is used up it takes
+        // slots from the others. One counter address serialises its atomics (about 85M/s), so a
+        // per-round atomic on one counter would cap the launch; a segment per XCD also keeps each
+        // XCD's L2 on one region of a sorted queue.
+        // fetch_chunk 0 claims exactly the slots the idle lanes need (the narrowest window of the
+        // queue in flight, one atomic per refill round); fetch_segments 1 or kFetchSegments.
+        const uint32_t waves = gridDim.x * (BLOCK / 64);
+        const uint32_t chunk = P.fetch_chunk ? max(64u, min(P.fetch_chunk, (count / max(1u, waves * 4u)) & ~63u)) : 0u;
+        const uint32_t nseg = P.fetch_segments > 1 ? kFetchSegments : 1u;
+        const uint32_t seg0 = blockIdx.x % nseg;
+        const bool simple = chunk == 0u && nseg == 1u;
+        uint32_t pool = 0, pool_end = 0; // wave-uniform: unclaimed slots [pool, pool_end)
+        bool drained = false;            // wave-uniform: every segment is used up
+        bool active = false, exhausted = false;
+        if (P.lanes != 0u) {
+            // every ray has a lane: wave w takes the slots [w lanes, w lanes + lanes) of the queue, with
+            // w counted XCD by XCD (block b runs on XCD b mod 8), so that each XCD has its own part
+            const uint32_t per_xcd = gridDim.x / kFetchSegments;
+            const uint32_t b = (blockIdx.x % kFetchSegments) * per_xcd + blockIdx.x / kFetchSegments;
+            const uint64_t w = (uint64_t)b * (BLOCK / 64) + (tid >> 6);
+            const uint64_t my = w * P.lanes + lane;
+            drained = exhausted = true;
+            if (lane < P.lanes && my < count) {
+                uint32_t bt, r;
+                Mode::locate(P, P.order ? P.order[my] : (uint32_t)my, bt, r);
+                start(P, bt, r);
+                active = true;
+            }
+        }
+        for (;;) {
+            const uint64_t need = __ballot(!active && !exhausted);
+            if (need) {
+                const uint32_t n_need = (uint32_t)__popcll(need);
+                const uint32_t rank = (uint32_t)__popcll(need & ((1ull << lane) - 1ull));
+                const uint32_t avail = pool_end - pool;
+                uint32_t my = rank < avail ? pool + rank : 0xFFFFFFFFu; // lanes served by the pool
+                if (simple) {
+                    // one counter, exactly the slots the idle lanes need
+                    const uint32_t leader = (uint32_t)__ffsll((long long)need) - 1u;
+                    uint32_t b = 0;
+                    if (lane == leader) b = atomicAdd(P.ray_counter, n_need);
+                    b = __builtin_amdgcn_readlane(b, (int)leader);
+                    my = b + rank;
+                    drained = b + n_need >= count;
+                } else if (avail >= n_need) {
+                    pool += n_need;
+                } else if (drained) {
+                    pool = pool_end;
+                } else {
+                    // refill: the leader claims a chunk of this XCD's segment, else of another one
+                    const uint32_t leader = (uint32_t)__ffsll((long long)need) - 1u;
+                    uint32_t nb = 0, ne = 0;
+                    if (lane == leader) {
+                        const uint32_t claim = chunk ? chunk : n_need - avail;
+                        for (uint32_t k = 0; k < nseg; k++) {
+                            const uint32_t s = (seg0 + k) % nseg;
+                            const uint32_t lo = (uint32_t)((uint64_t)count * s / nseg);
+                            const uint32_t hi = (uint32_t)((uint64_t)count * (s + 1) / nseg);
+                            if (lo == hi) continue;
+                            const uint32_t b = atomicAdd(P.ray_counter + s * kCounterStride, claim);
+                            if (b < hi - lo) {
+                                nb = lo + b;
+                                ne = lo + min(b + claim, hi - lo);
+                                break;
+                            }
+                        }
+                    }
+                    nb = __builtin_amdgcn_readlane(nb, (int)leader); // wave-uniform from here on
+                    ne = __builtin_amdgcn_readlane(ne, (int)leader);
+                    drained = nb == ne;
+                    if (rank >= avail && rank - avail < ne - nb) my = nb + (rank - avail);
+                    pool = nb + min(n_need - avail, ne - nb);
+                    pool_end = ne;
+                }
+                if (!active && !exhausted) {
+                    if (my < count) {
+                        uint32_t b, r;
+                        Mode::locate(P, P.order ? P.order[my] : my, b, r); // sorted queue: fetch in key order
+                        start(P, b, r);
+                        active = true;
+                    } else if (drained) {
+                        exhausted = true; // no slot left in any segment (else: retry next round)
+                    }
+                }
+            }
+            if (!__any(active)) break;
+            if (COUNT && lane == (uint32_t)__ffsll((long long)__ballot(1)) - 1u) rounds++;
+            run(P, active, !drained);
+            if (active && finished()) {
+                if (!COUNT) write(P); // the counting form has no output buffers (out is null)
+                active = false;
+            }
+        }
+        return rounds;
     }
 };
 
