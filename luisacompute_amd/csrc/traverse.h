@@ -164,9 +164,10 @@ __device__ __forceinline__ uint32_t intersect_node(const RaySetup &r, const uint
     const uint32_t nx0 = nx ? w3.z : w2.x, nx1 = nx ? w3.w : w2.y, fx0 = nx ? w2.x : w3.z, fx1 = nx ? w2.y : w3.w;
     const uint32_t ny0 = ny ? w4.x : w2.z, ny1 = ny ? w4.y : w2.w, fy0 = ny ? w2.z : w4.x, fy1 = ny ? w2.w : w4.y;
     const uint32_t nz0 = nz ? w4.z : w3.x, nz1 = nz ? w4.w : w3.y, fz0 = nz ? w3.x : w4.z, fz1 = nz ? w3.y : w4.w;
-    uint32_t hits = 0;
+    tcull += 0.0f; // -0 to 0: -0 less 0 would read as a miss below
+    uint32_t miss = 0;
 #pragma unroll
-    for (int s = 0; s < 8; s++) {
+    for (int s = 7; s >= 0; s--) {
         const int k = s & 3;
         const uint32_t wnx = s < 4 ? nx0 : nx1, wfx = s < 4 ? fx0 : fx1;
         const uint32_t wny = s < 4 ? ny0 : ny1, wfy = s < 4 ? fy0 : fy1;
@@ -180,9 +181,11 @@ __device__ __forceinline__ uint32_t intersect_node(const RaySetup &r, const uint
         float tfz = __builtin_fmaf(plane_1024(plane_halves(wfz, pair), hi), a[2], bf[2]);
         float tn = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, tmin));
         float tf = fminf(fminf(tfx, tfy), fminf(tfz, tcull));
-        if (tn <= tf) hits |= 1u << s;
+        // the sign of the difference shifted into the mask: a compare, a select and half an or otherwise
+        // (an infinity less itself is a positive NaN here: a hit)
+        miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(tf - tn), 31u);
     }
-    return hits;
+    return ~miss & 0xFFu;
 }
 
 __device__ __forceinline__ void xform_point(const float m[12], const float p[3], float out[3]) {
