@@ -110,6 +110,7 @@ struct TraceParams {
                              // hold a ray (0: refill only after `steps` steps)
     uint32_t lanes;          // 0: waves claim slots as they go; else wave w takes the `lanes` slots from
                              // w x lanes on, and no others (trace_grid)
+    uint32_t octets;         // eight lanes per ray (then lanes <= 8 rays per wave, workgroups of 64)
 };
 
 // ---- kernels (radix.hip) ----
@@ -298,8 +299,9 @@ hipError_t noalloc_scratch_lookup(void **device_ptr);
 struct TraceGrid {
     int grid;
     uint32_t lanes;
+    bool octets;
 };
-TraceGrid trace_grid(uint64_t count, int block, int blocks_per_cu, int cu_count);
+TraceGrid trace_grid(uint64_t count, int block, int blocks_per_cu, int cu_count, bool octets);
 hipError_t trace_launch(const TraceParams &P, hipStream_t stream, bool any, bool two, bool count, int grid, int block,
                         int slds);
 

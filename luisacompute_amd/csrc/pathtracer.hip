@@ -833,7 +833,7 @@ static int run_wave(Device *dev, hipStream_t s, Workspace &W, const PtBinding &B
     const bool two = Bd.two;
     const int bpc_c = cc.blocks_per_cu > 0 ? cc.blocks_per_cu : trace_blocks_per_cu(false, two, false, cc.block, cc.slds);
     const int bpc_a = ca.blocks_per_cu > 0 ? ca.blocks_per_cu : trace_blocks_per_cu(true, two, false, ca.block, ca.slds);
-    const TraceGrid tg_c = trace_grid(cap, cc.block, bpc_c, dev->cu_count), tg_a = trace_grid(cap, ca.block, bpc_a, dev->cu_count);
+    const TraceGrid tg_c = trace_grid(cap, cc.block, bpc_c, dev->cu_count, true), tg_a = trace_grid(cap, ca.block, bpc_a, dev->cu_count, true);
     const int grid_c = tg_c.grid, grid_a = tg_a.grid;
     const uint32_t sd_c = Bd.stack_need > (uint32_t)cc.slds ? Bd.stack_need - cc.slds : 0u;
     const uint32_t sd_a = Bd.stack_need > (uint32_t)ca.slds ? Bd.stack_need - ca.slds : 0u;
@@ -897,6 +897,7 @@ static int run_wave(Device *dev, hipStream_t s, Workspace &W, const PtBinding &B
             P.error = dev->error;
             P.hit_record = 1u;
             P.lanes = tg_c.lanes;
+            P.octets = tg_c.octets ? 1u : 0u;
             hipError_t e = trace_launch(P, s, false, two, false, grid_c, cc.block, cc.slds);
             if (e != hipSuccess) return e;
             hipLaunchKernelGGL(k_pt_counters, dim3(1), dim3(64), 0, s, Q, cur, nxt, counts, 0);
@@ -912,6 +913,7 @@ static int run_wave(Device *dev, hipStream_t s, Workspace &W, const PtBinding &B
             A.refill_below = ca.refill_below;
             A.hit_record = 0u;
             A.lanes = tg_a.lanes;
+            A.octets = tg_a.octets ? 1u : 0u;
             e = trace_launch(A, s, true, two, false, grid_a, ca.block, ca.slds);
             if (e != hipSuccess) return e;
             hipLaunchKernelGGL(k_pt_counters, dim3(1), dim3(64), 0, s, Q, cur, nxt, counts, 1);

@@ -1688,11 +1688,13 @@ static int trace_launch_batches(Device *dev, Accel *a, hipStream_t s, const lc_h
     if (grc != LC_HIP_OK) return grc;
     std::lock_guard<std::mutex> dl(dev->mu);
     const TraceConfig &cfg = dev->cfg[any ? 1 : 0];
-    // the counting form runs the timed form's grid (same waves, same queue hand-out)
+    // the counting form runs the timed form's grid (same waves, same queue hand-out), but with one lane
+    // per ray also where the timed form takes eight (whose visits and tests differ a little in order)
     int bpc = cfg.blocks_per_cu > 0 ? cfg.blocks_per_cu : trace_blocks_per_cu(any, two, false, cfg.block, cfg.slds);
-    const TraceGrid tg = trace_grid(total, cfg.block, bpc, dev->cu_count);
+    const TraceGrid tg = trace_grid(total, cfg.block, bpc, dev->cu_count, !counting);
     const int grid = tg.grid;
     P.lanes = tg.lanes;
+    P.octets = tg.octets ? 1u : 0u;
     P.spill_depth = stack_need > (uint32_t)cfg.slds ? stack_need - (uint32_t)cfg.slds : 0u;
     size_t spill_bytes = (size_t)grid * cfg.block * P.spill_depth * sizeof(uint2);
     StreamScratch *S = stream_scratch(dev, s);
@@ -1937,7 +1939,7 @@ int lc_hip_accel_trace_closest_noalloc(uint64_t device, uint64_t stream, uint64_
     std::lock_guard<std::mutex> dl(dev->mu);
     const TraceConfig &cfg = dev->cfg[0];
     const int bpc = cfg.blocks_per_cu > 0 ? cfg.blocks_per_cu : trace_blocks_per_cu(false, two, false, cfg.block, cfg.slds);
-    TraceGrid tg = trace_grid(ray_count, cfg.block, bpc, dev->cu_count);
+    TraceGrid tg = trace_grid(ray_count, cfg.block, bpc, dev->cu_count, true);
     uint64_t grid = (uint64_t)tg.grid;
     P.spill_depth = stack_need > (uint32_t)cfg.slds ? stack_need - (uint32_t)cfg.slds : 0u;
     const size_t spill_per_block = (size_t)cfg.block * P.spill_depth * sizeof(uint2);
@@ -1949,8 +1951,10 @@ int lc_hip_accel_trace_closest_noalloc(uint64_t device, uint64_t stream, uint64_
     if (spill_per_block && grid > spill_cap / spill_per_block) { // a smaller grid: waves claim slots as they go
         grid = spill_cap / spill_per_block;
         tg.lanes = 0u;
+        tg.octets = false;
     }
     P.lanes = tg.lanes;
+    P.octets = tg.octets ? 1u : 0u;
     static_assert(576 + 2 * sizeof(unsigned long long) <= kNoAllocWordsBytes, "no-allocation words");
     char *base = static_cast<char *>(dev->noalloc_scratch);
     P.ray_counter = reinterpret_cast<uint32_t *>(base);
@@ -2028,7 +2032,7 @@ int lc_hip_accel_query(uint64_t device, uint64_t stream, uint64_t accel, uint64_
         const uint64_t want = ((uint64_t)ray_count + block - 1) / block;
         grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)bpc * cus, want));
     } else {
-        const TraceGrid tg = trace_grid(ray_count, block, bpc, cus);
+        const TraceGrid tg = trace_grid(ray_count, block, bpc, cus, false);
         grid = tg.grid;
         P.lanes = tg.lanes;
     }

@@ -22,6 +22,7 @@
 
 #include "lc_hip_bvh.h"
 #include "lc_hip_internal.h"
+#include "oct_walker.h"
 #include "wave_walker.h"
 
 // Working memory of lc_hip_accel_trace_closest_noalloc: the launch's slot counters, error word
@@ -78,6 +79,27 @@ void k_trace(const TraceParams P) {
             if (lane == 0) atomicAdd(reinterpret_cast<unsigned long long *>(P.stats) + k, (unsigned long long)v[k]);
         }
     }
+}
+
+// Eight lanes per ray, P.lanes rays per wave (trace_grid); every ray of the launch has its lanes.
+template<bool ANY, bool TWO>
+__global__ __launch_bounds__(64) void k_trace_oct(const TraceParams P) {
+    __shared__ uint2 stk[trav::kOctStack][8];
+    const uint32_t count = P.count_ptr ? min(*P.count_ptr, P.count) : P.count;
+    trav::OctWalker<ANY, TWO> W;
+    W.stk = stk;
+    W.k = threadIdx.x & 7u;
+    W.group = threadIdx.x >> 3;
+    // waves XCD by XCD, as in WaveWalker::trace_queue
+    const uint32_t w = (blockIdx.x % kFetchSegments) * (gridDim.x / kFetchSegments) + blockIdx.x / kFetchSegments;
+    const uint64_t my = (uint64_t)w * P.lanes + W.group;
+    if (W.group >= P.lanes || my >= count) return;
+    W.start(P, P.order ? P.order[my] : (uint32_t)my);
+    for (;;) {
+        if (((W.g_mask & 0xFFu) == 0u || (TWO && W.t_mask != 0u)) && !W.next_group(P)) break;
+        W.visit(P);
+    }
+    if (W.k == 0u) W.write(P);
 }
 
 __global__ void k_zero_counter(uint32_t *c) {
@@ -138,26 +160,44 @@ int trace_blocks_per_cu(bool any, bool two, bool count, int block, int slds) {
 }
 
 // A launch whose rays all fit the lanes that can be resident hands them out once, without slot
-// counters (and without the launch that clears them). When that leaves SIMDs without a wave, waves
-// take fewer rays instead, down to kMinLanes: a wave lasts as long as its slowest ray plus the
-// triangle steps of the others, one step after another, each a memory latency (4,096 rays on
-// 81,920 triangles: 98 us with 64 rays per wave, 60 with 4; 16 per wave 65).
-TraceGrid trace_grid(uint64_t count, int block, int blocks_per_cu, int cu_count) {
-    constexpr uint32_t kMinLanes = 4;
+// counters (and without the launch that clears them).
+//  - Eight lanes per ray (k_trace_oct) while kOctWaves waves per SIMD hold every ray: 65,536 rays on
+//    256 CUs. Measured, one ray per lane against eight lanes per ray, 1 M triangles of a soup,
+//    closest hit: 1,024 rays 120 -> 70 us, 16,384 172 -> 103, 32,768 175 -> 121, 49,152 186 -> 128,
+//    65,536 185 -> 183, 98,304 188 -> 214; any hit 65,536 143 -> 114; 81,920 triangles of a
+//    sphere, 16,384 rays 85 -> 41, 65,536 100 -> 71. The eight lanes do the node decode eight times,
+//    so the form loses once the SIMDs have enough waves to be bound by VALU issue.
+//  - Otherwise one ray per lane; when that leaves SIMDs without a wave, waves take fewer rays (down
+//    to kMinLanes: nearest-commit queries, and traces that count their work): a wave lasts as long
+//    as its slowest ray plus the triangle steps of the others, one step after another, each a
+//    memory latency.
+TraceGrid trace_grid(uint64_t count, int block, int blocks_per_cu, int cu_count, bool octets) {
+    constexpr uint32_t kMinLanes = 4, kOctWaves = 8;
     const uint64_t cus = (uint64_t)std::max(1, cu_count);
     const uint64_t most = (uint64_t)std::max(1, blocks_per_cu) * cus;
     const uint64_t waves_per_block = (uint64_t)(block / 64);
-    if (count > most / kFetchSegments * kFetchSegments * (uint64_t)block) return {(int)most, 0u};
+    if (count > most / kFetchSegments * kFetchSegments * (uint64_t)block) return {(int)most, 0u, false};
     const uint64_t simds = 4u * cus;
+    if (octets && count <= simds * kOctWaves * 8u) {
+        uint32_t rays = 1; // per wave
+        while (rays < 8u && (count + rays - 1) / rays > simds) rays *= 2u;
+        return {(int)(((count + rays - 1) / rays + kFetchSegments - 1) / kFetchSegments * kFetchSegments), rays, true};
+    }
     uint32_t lanes = kMinLanes;
     while (lanes < 64u && (count + lanes - 1) / lanes > simds) lanes *= 2u;
     uint64_t grid = ((count + lanes - 1) / lanes + waves_per_block - 1) / waves_per_block;
     grid = (grid + kFetchSegments - 1) / kFetchSegments * kFetchSegments; // k_trace counts waves XCD by XCD
-    return {(int)grid, lanes};
+    return {(int)grid, lanes, false};
 }
 
 hipError_t trace_launch(const TraceParams &P, hipStream_t stream, bool any, bool two, bool count, int grid, int block,
                         int slds) {
+    if (P.octets != 0u && !count) {
+        const auto k = any ? (two ? k_trace_oct<true, true> : k_trace_oct<true, false>)
+                           : (two ? k_trace_oct<false, true> : k_trace_oct<false, false>);
+        hipLaunchKernelGGL(k, dim3(grid), dim3(64), 0, stream, P);
+        return hipGetLastError();
+    }
     if (P.lanes == 0u)
         hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, stream, P.ray_counter);
     if (any) {

@@ -1,7 +1,8 @@
-"""GPU tests of how a trace launch hands out its rays (trace_grid, k_trace): launches that give every
-ray a lane, with 4 to 64 rays per wave, against larger ones whose waves claim queue slots, around the
-sizes where the form changes, in queue order and sorted. Every size gives the hits of the large launch,
-ray by ray, and writes nothing past its last ray."""
+"""GPU tests of how a trace launch hands out its rays (trace_grid, k_trace, k_trace_oct): launches
+that give every ray eight lanes, with 1 to 8 rays per wave, or one lane, with 64 rays per wave,
+against larger ones whose waves claim queue slots, around the sizes where the form changes, in queue
+order and sorted. Every size gives the hits of the large launch, ray by ray, and writes nothing past
+its last ray."""
 import numpy as np
 import pytest
 
@@ -12,7 +13,7 @@ from parity import compare_any, compare_closest
 
 pytestmark = pytest.mark.gpu
 N = 420000  # more rays than lanes are resident (256 CUs x 24 waves x 64)
-SIZES = (1, 3, 4, 5, 63, 64, 65, 4095, 4096, 4097, 8193, 65535, 65537, 262143, 262144, 262145, 393216, 393217, N)
+SIZES = (1, 3, 4, 5, 63, 64, 65, 1023, 1025, 2049, 4095, 4096, 4097, 8191, 8193, 65535, 65536, 65537, 262143, 262144, 262145, 393216, 393217, N)
 
 
 @pytest.fixture(scope="module", params=("one", "two"))

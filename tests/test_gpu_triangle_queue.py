@@ -2,7 +2,9 @@
 can go wrong: more triangles per step than the queue holds, leaves of one and of three triangles,
 last steps that fill only part of a wave, hits at equal distances and at zero, and instances that
 are left, skipped or masked while pairs are queued. Everything is compared with the oracle bit for
-bit (hits do not depend on the order in which triangles are tested)."""
+bit (hits do not depend on the order in which triangles are tested). The rays are traced as they are,
+a launch with eight lanes per ray (oct_walker.h), and repeated past the size at which waves take one
+ray per lane and share a queue."""
 import numpy as np
 import pytest
 
@@ -34,6 +36,16 @@ def _rays(n, rng, z=-1.0, t_min=0.0):
     return r
 
 
+def _one_lane_per_ray(device, stream, accel, rays, mask=0xFF):
+    """The rays repeated past 65,536: hits of the first round, each later round the same."""
+    reps = 70000 // len(rays) + 1
+    many = np.tile(rays, reps)
+    closest, any_hit = host.trace_closest(device, stream, accel, many, mask), host.trace_any(device, stream, accel, many, mask)
+    closest, any_hit = closest.reshape(reps, -1), np.asarray(any_hit).reshape(reps, -1)
+    assert (closest.view(np.uint32) == closest[:1].view(np.uint32)).all() and (any_hit == any_hit[:1]).all()
+    return closest[0], any_hit[0]
+
+
 def _check(device, stream, accel, scene, rays, ties_exact=True):
     g = host.trace_closest(device, stream, accel, rays)
     f = lc.rays_as_floats(rays)
@@ -42,7 +54,11 @@ def _check(device, stream, accel, scene, rays, ties_exact=True):
     if ties_exact:  # equal distances: the smaller (instance, primitive), as in the oracle
         np.testing.assert_array_equal(g["prim"], ref["prim"])
         np.testing.assert_array_equal(g["inst"], ref["inst"])
-    compare_any(host.trace_any(device, stream, accel, rays), scene.trace_any(f))
+    any_hit = host.trace_any(device, stream, accel, rays)
+    compare_any(any_hit, scene.trace_any(f))
+    closest2, any2 = _one_lane_per_ray(device, stream, accel, rays)
+    np.testing.assert_array_equal(closest2.view(np.uint32), g.view(np.uint32))
+    np.testing.assert_array_equal(any2, any_hit)
     return g
 
 
@@ -103,5 +119,9 @@ def test_instances_left_skipped_and_masked(device, stream, count, mask):
     scene.commit()
     rays = lc.rays_box_sphere(5001, initseq=91 + count, lo=-20.0, hi=20.0)
     f = lc.rays_as_floats(rays)
-    compare_closest(host.trace_closest(device, stream, accel, rays, mask), scene.trace_closest2(f, mask), rays)
-    compare_any(host.trace_any(device, stream, accel, rays, mask), scene.trace_any(f, mask))
+    closest, any_hit = host.trace_closest(device, stream, accel, rays, mask), host.trace_any(device, stream, accel, rays, mask)
+    compare_closest(closest, scene.trace_closest2(f, mask), rays)
+    compare_any(any_hit, scene.trace_any(f, mask))
+    closest2, any2 = _one_lane_per_ray(device, stream, accel, rays, mask)
+    np.testing.assert_array_equal(closest2.view(np.uint32), closest.view(np.uint32))
+    np.testing.assert_array_equal(any2, any_hit)
