@@ -111,6 +111,8 @@ struct TraceParams {
     uint32_t lanes;          // 0: waves claim slots as they go; else wave w takes the `lanes` slots from
                              // w x lanes on, and no others (trace_grid)
     uint32_t octets;         // eight lanes per ray (then lanes <= 8 rays per wave, workgroups of 64)
+    uint32_t simds;          // with count_ptr: SIMDs of the GPU, for the choice of eight lanes per ray
+                             // once the count is known (0: none)
 };
 
 // ---- kernels (radix.hip) ----

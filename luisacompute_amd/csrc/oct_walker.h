@@ -254,5 +254,22 @@ struct OctWalker {
     }
 };
 
+// Wave w of the launch traces the `rays` queue slots from w x rays on.
+template<bool ANY, bool TWO>
+__device__ __forceinline__ void trace_octets(const TraceParams &P, uint2 (*stk)[8], uint32_t w, uint32_t rays, uint32_t count) {
+    OctWalker<ANY, TWO> W;
+    W.stk = stk;
+    W.k = threadIdx.x & 7u;
+    W.group = threadIdx.x >> 3;
+    const uint64_t my = (uint64_t)w * rays + W.group;
+    if (W.group >= rays || my >= count) return;
+    W.start(P, P.order ? P.order[my] : (uint32_t)my);
+    for (;;) {
+        if (((W.g_mask & 0xFFu) == 0u || (TWO && W.t_mask != 0u)) && !W.next_group(P)) break;
+        W.visit(P);
+    }
+    if (W.k == 0u) W.write(P);
+}
+
 } // namespace trav
 } // namespace lchip

@@ -898,6 +898,7 @@ static int run_wave(Device *dev, hipStream_t s, Workspace &W, const PtBinding &B
             P.hit_record = 1u;
             P.lanes = tg_c.lanes;
             P.octets = tg_c.octets ? 1u : 0u;
+            P.simds = 4u * (uint32_t)std::max(1, dev->cu_count);
             hipError_t e = trace_launch(P, s, false, two, false, grid_c, cc.block, cc.slds);
             if (e != hipSuccess) return e;
             hipLaunchKernelGGL(k_pt_counters, dim3(1), dim3(64), 0, s, Q, cur, nxt, counts, 0);
@@ -914,6 +915,7 @@ static int run_wave(Device *dev, hipStream_t s, Workspace &W, const PtBinding &B
             A.hit_record = 0u;
             A.lanes = tg_a.lanes;
             A.octets = tg_a.octets ? 1u : 0u;
+            A.simds = P.simds;
             e = trace_launch(A, s, true, two, false, grid_a, ca.block, ca.slds);
             if (e != hipSuccess) return e;
             hipLaunchKernelGGL(k_pt_counters, dim3(1), dim3(64), 0, s, Q, cur, nxt, counts, 1);

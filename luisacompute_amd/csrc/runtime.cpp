@@ -1695,6 +1695,7 @@ static int trace_launch_batches(Device *dev, Accel *a, hipStream_t s, const lc_h
     const int grid = tg.grid;
     P.lanes = tg.lanes;
     P.octets = tg.octets ? 1u : 0u;
+    P.simds = count_ptr ? 4u * (uint32_t)std::max(1, dev->cu_count) : 0u;
     P.spill_depth = stack_need > (uint32_t)cfg.slds ? stack_need - (uint32_t)cfg.slds : 0u;
     size_t spill_bytes = (size_t)grid * cfg.block * P.spill_depth * sizeof(uint2);
     StreamScratch *S = stream_scratch(dev, s);

@@ -67,6 +67,25 @@ void k_trace(const TraceParams P) {
     __shared__ trav::WaveShared<ANY, BLOCK, SLDS> shared;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t count = P.count_ptr ? min(*P.count_ptr, P.count) : P.count;
+    if constexpr (BLOCK == 64 && !COUNT) {
+        // A queue counted on the device that turns out short: eight lanes per ray, in as many waves as
+        // trace_grid would take and a second round or part of one, spread over the XCDs (the last depths of
+        // a path-traced wave, whose launches are sized for its first: closest 160 -> 50 us, any 140 -> 27).
+        // The limits, 51,200 and 81,920 rays for two levels on 256 CUs, lie within the sizes at which eight
+        // lanes per ray are faster on every scene measured (trace_grid).
+        constexpr uint32_t kRays = ANY ? 16u : 10u; // per resident wave
+        const uint32_t blocks = gridDim.x & ~(kFetchSegments - 1u);
+        if (P.simds != 0u && count <= kRays * blocks) {
+            uint32_t rays = 1u;
+            while (rays < 8u && (count + rays - 1u) / rays > min(P.simds, blocks)) rays *= 2u;
+            const uint32_t per_xcd = min(blocks, (count + rays - 1u) / rays + kFetchSegments - 1u) / kFetchSegments;
+            if (blockIdx.x >= per_xcd * kFetchSegments) return;
+            for (uint32_t w = (blockIdx.x % kFetchSegments) * per_xcd + blockIdx.x / kFetchSegments; w * rays < count;
+                 w += per_xcd * kFetchSegments)
+                trav::trace_octets<ANY, TWO>(P, reinterpret_cast<uint2 (*)[8]>(&shared.stk[0][0]), w, rays, count);
+            return;
+        }
+    }
     trav::WaveWalker<ANY, TWO, COUNT, BLOCK, SLDS> W;
     W.init(P, &shared, tid);
 
@@ -86,20 +105,9 @@ template<bool ANY, bool TWO>
 __global__ __launch_bounds__(64) void k_trace_oct(const TraceParams P) {
     __shared__ uint2 stk[trav::kOctStack][8];
     const uint32_t count = P.count_ptr ? min(*P.count_ptr, P.count) : P.count;
-    trav::OctWalker<ANY, TWO> W;
-    W.stk = stk;
-    W.k = threadIdx.x & 7u;
-    W.group = threadIdx.x >> 3;
     // waves XCD by XCD, as in WaveWalker::trace_queue
     const uint32_t w = (blockIdx.x % kFetchSegments) * (gridDim.x / kFetchSegments) + blockIdx.x / kFetchSegments;
-    const uint64_t my = (uint64_t)w * P.lanes + W.group;
-    if (W.group >= P.lanes || my >= count) return;
-    W.start(P, P.order ? P.order[my] : (uint32_t)my);
-    for (;;) {
-        if (((W.g_mask & 0xFFu) == 0u || (TWO && W.t_mask != 0u)) && !W.next_group(P)) break;
-        W.visit(P);
-    }
-    if (W.k == 0u) W.write(P);
+    trav::trace_octets<ANY, TWO>(P, stk, w, P.lanes, count);
 }
 
 __global__ void k_zero_counter(uint32_t *c) {

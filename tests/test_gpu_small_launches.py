@@ -63,14 +63,21 @@ def test_every_size_gives_the_same_hits(device, stream, scene, block, sort):
             np.testing.assert_array_equal(occluded[:n], any_hit[:n])
             assert (hits[n:].view(np.uint8) == 0xA5).all() and (occluded[n:] == 0xA5).all()
         # the length read on the device: fewer rays than the launch has lanes for
-        for capacity, n in ((4096, 0), (4096, 77), (65537, 1000), (N, 5000)):
+        for capacity, n in ((4096, 0), (4096, 77), (65537, 1000), (N, 0), (N, 3), (N, 5000), (N, 40961),
+                            (N, 51200), (N, 51201), (N, 61441), (N, 81921), (N, 98304), (N, 98305)):
             print(f"[launch] block {block} sort {sort} capacity {capacity} rays {n}", flush=True)
             hits = np.full((N + 16) * 24, 0xA5, np.uint8).view(lc.HIT_DTYPE)
             stream << hb.copy_from(hits) << count.copy_from(np.array([n], np.uint32))
             accel.trace_closest_indirect(stream, rb, hb, count, capacity=capacity)
             stream << hb.copy_to(hits) << lc.synchronize()
+            occluded = blank.copy()
+            stream << ab.copy_from(occluded)
+            accel.trace_any_indirect(stream, rb, ab, count, capacity=capacity)
+            stream << ab.copy_to(occluded) << lc.synchronize()
             np.testing.assert_array_equal(hits[:n].view(np.uint32), closest[:n].view(np.uint32))
             assert (hits[n:].view(np.uint8) == 0xA5).all()
+            np.testing.assert_array_equal(occluded[:n], any_hit[:n])
+            assert (occluded[n:] == 0xA5).all()
     finally:
         for k, (c, srt) in saved.items():
             device.set_trace_config(k, c["block"], c["lds_stack"], c["steps"], c["blocks_per_cu"])
