@@ -6,7 +6,7 @@
 // cpu/accel.rs:205-260). Neither reference path has a software builder; the steps here are:
 //   1. centroid bounds (wave64 shuffle reduction + one atomic per block); primitive boxes are
 //      stored once, in input order, by the Morton kernel;
-//   2. 30-bit Morton codes (10 bits per axis), radix sort of (code, primitive id) (rocPRIM);
+//   2. 30-bit Morton codes (10 bits per axis), radix sort of (code, primitive id) (radix.hip);
 //   3. binary radix tree from the sorted codes alone (Karras 2012), equal codes ordered by index;
 //   4. node boxes bottom-up in phases whose child handoffs stay inside one workgroup (so they
 //      only need workgroup-scope ordering -- an agent-scope release/acquire writes back and

@@ -3,8 +3,8 @@
 // Replaces the reference's lc_accel_trace_closest / lc_accel_trace_any
 // (src/backends/cuda/cuda_builtin/cuda_device_resource.h:1783-1829, OptiX hardware traversal)
 // with the observable semantics of the CPU backend's AccelImpl::trace_closest / trace_any
-// (src/rust/luisa_compute_backend_impl/src/cpu/accel.rs:449-535); the per-ray traversal is the
-// Walker of traverse.h.
+// (src/rust/luisa_compute_backend_impl/src/cpu/accel.rs:449-535); the traversal is that of
+// wave_walker.h (one ray per lane) or oct_walker.h (eight lanes per ray, for launches of few rays).
 //
 // Launch design (wave64): a persistent grid; a wave hands rays to its idle lanes from a pool of
 // queue slots it claims in chunks (per-XCD queue segments, below), runs `steps` traversal steps,
@@ -58,9 +58,9 @@ hipError_t noalloc_scratch_lookup(void **device_ptr) {
 
 // Template parameters: ANY (trace_any), TWO (TLAS + BLAS; otherwise one instance's BLAS),
 // COUNT (count node visits / triangle tests), BLOCK threads, SLDS stack entries in LDS.
-// With the 8-entry LDS stack the single-level forms fit 7 (any-hit, <= 72 VGPRs) and 6
-// (closest-hit, <= 80 VGPRs) waves per SIMD without spilling; the hint keeps the register
-// allocator there (deeper LDS stacks are limited by LDS first).
+// With the 8-entry LDS stack the single-level forms fit 6 (<= 80 VGPRs) and the two-level forms 5
+// (<= 96 VGPRs) waves per SIMD without spilling; the hint keeps the register allocator there
+// (deeper LDS stacks are limited by LDS first).
 template<bool ANY, bool TWO, bool COUNT, int BLOCK, int SLDS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(SLDS == 8 ? (TWO ? 5 : 6) : 1)))
 void k_trace(const TraceParams P) {

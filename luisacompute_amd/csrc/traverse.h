@@ -123,8 +123,6 @@ __device__ __forceinline__ uint32_t permute8(uint32_t m, uint32_t f) {
     return m;
 }
 
-__device__ __forceinline__ float ubyte(uint32_t w, int k) { return (float)((w >> (8 * k)) & 0xFFu); }
-
 // Quantised planes as IEEE halves: byte q of a plane word becomes the low byte of a half whose high
 // byte is 0x64, i.e. the half 1024 + q (exact). One byte permute makes the halves of two planes,
 // and a fused multiply-add takes a half operand as it is (v_fma_mix_f32), so a plane costs half a
@@ -223,7 +221,8 @@ __device__ __forceinline__ bool nearer(float t, uint32_t inst, uint32_t prim, fl
     return inst != b_inst ? inst < b_inst : prim < b_prim;
 }
 
-// One ray's traversal. ANY: stop at the first hit; TWO: TLAS + BLAS (otherwise the single
+// One ray's traversal (the path tracer's megakernel; trace launches use the walkers of wave_walker.h and
+// oct_walker.h). ANY: stop at the first hit; TWO: TLAS + BLAS (otherwise the single
 // instance of G); COUNT: count node visits and triangle tests. The stack's LDS part is the
 // column `tid` of an [SLDS][BLOCK] array; entries beyond SLDS go to `spill`.
 template<bool ANY, bool TWO, bool COUNT, int BLOCK, int SLDS>
@@ -444,16 +443,6 @@ struct Walker {
             }
         }
         return false;
-    }
-
-    // Closest-hit record (24-B SurfaceHit as three uint2). The padding word after t carries the
-    // leaf record index when `record` is set (queues internal to the path tracer), else 0.
-    __device__ __forceinline__ void write_hit(uint2 *h, bool record) const {
-        const bool hit = b_prim != 0xFFFFFFFFu;
-        const uint32_t t_bits = hit ? __float_as_uint(t_best) : __float_as_uint(tmax);
-        h[0] = make_uint2(hit ? b_inst : 0xFFFFFFFFu, b_prim);
-        h[1] = make_uint2(hit ? __float_as_uint(bu) : 0u, hit ? __float_as_uint(bv) : 0u);
-        h[2] = make_uint2(t_bits, (hit && record) ? b_rec : 0u);
     }
 };
 
