@@ -322,6 +322,15 @@ struct TraceConfig {
     uint32_t refill_below = 48;
 };
 
+// The step policy of a launch of a trace kind (TraceParams or QueryParams): all of it from that kind's
+// configuration, also where the launch's other parameters are those of another kind.
+template<class Params>
+inline void set_step_policy(Params &P, const TraceConfig &cfg) {
+    P.steps = cfg.steps;
+    P.tri_quarters = cfg.tri_quarters;
+    P.refill_below = cfg.refill_below;
+}
+
 struct TimingStat {
     double total_ms = 0.0;
     uint64_t launches = 0;

@@ -888,11 +888,9 @@ static int run_wave(Device *dev, hipStream_t s, Workspace &W, const PtBinding &B
             P.geo = Bd.G;
             P.spill = W.spill;
             P.spill_depth = sd_c;
-            P.steps = cc.steps;
+            set_step_policy(P, cc);
             P.fetch_chunk = opt.fetch_chunk;
             P.fetch_segments = opt.fetch_segments;
-            P.tri_quarters = cc.tri_quarters;
-            P.refill_below = cc.refill_below;
             P.stats = nullptr;
             P.error = dev->error;
             P.hit_record = 1u;
@@ -910,8 +908,7 @@ static int run_wave(Device *dev, hipStream_t s, Workspace &W, const PtBinding &B
             A.count_ptr = Q.ctr + 3;
             A.ray_counter = Q.ctr + kCtrAny;
             A.spill_depth = sd_a;
-            A.steps = ca.steps;
-            A.refill_below = ca.refill_below;
+            set_step_policy(A, ca);
             A.hit_record = 0u;
             A.lanes = tg_a.lanes;
             A.octets = tg_a.octets ? 1u : 0u;

@@ -1705,11 +1705,9 @@ static int trace_launch_batches(Device *dev, Accel *a, hipStream_t s, const lc_h
     P.ray_counter = S->ray_counter;
     P.error = S->error;
     P.stats = S->stats;
-    P.steps = cfg.steps;
+    set_step_policy(P, cfg);
     P.fetch_chunk = cfg.fetch_chunk;
     P.fetch_segments = cfg.fetch_segments;
-    P.tri_quarters = cfg.tri_quarters;
-    P.refill_below = cfg.refill_below;
     if (counting) LC_HIP_TRY(hipMemsetAsync(S->stats, 0, 5 * sizeof(unsigned long long), s));
     // per-ray results do not depend on the order; the counting form traverses the same sorted
     // queue as the timed form, so its node / triangle totals describe that launch. Queues counted
@@ -1962,11 +1960,9 @@ int lc_hip_accel_trace_closest_noalloc(uint64_t device, uint64_t stream, uint64_
     P.error = reinterpret_cast<uint32_t *>(base) + kRayCounterWords;
     P.stats = reinterpret_cast<unsigned long long *>(base + 576);
     P.spill = reinterpret_cast<uint2 *>(base + kNoAllocWordsBytes);
-    P.steps = cfg.steps;
+    set_step_policy(P, cfg);
     P.fetch_chunk = cfg.fetch_chunk;
     P.fetch_segments = cfg.fetch_segments;
-    P.tri_quarters = cfg.tri_quarters;
-    P.refill_below = cfg.refill_below;
     const hipError_t e = trace_launch(P, s, false, two, false, (int)grid, cfg.block, cfg.slds);
     if (e != hipSuccess) return hip_fail(e, "trace launch");
     return LC_HIP_OK;
@@ -2037,11 +2033,9 @@ int lc_hip_accel_query(uint64_t device, uint64_t stream, uint64_t accel, uint64_
         grid = tg.grid;
         P.lanes = tg.lanes;
     }
-    P.steps = cfg.steps;
+    set_step_policy(P, cfg);
     P.fetch_chunk = cfg.fetch_chunk;
     P.fetch_segments = cfg.fetch_segments;
-    P.tri_quarters = cfg.tri_quarters;
-    P.refill_below = cfg.refill_below;
     const uint32_t slds = (uint32_t)query_lds_entries();
     P.spill_depth = stack_need > slds ? stack_need - slds : 0u;
     StreamScratch *S = stream_scratch(dev, s);
