@@ -737,16 +737,18 @@ __global__ __launch_bounds__(64) void k_sah_clusters(const uint32_t *entries, co
             }
             s_box[0][lane] = lo.x; s_box[1][lane] = lo.y; s_box[2][lane] = lo.z;
             s_box[3][lane] = hi.x; s_box[4][lane] = hi.y; s_box[5][lane] = hi.z;
-            // centroids as ordered integers whose low 6 bits are the lane, so no two are equal
-            key[0] = (ord_u32(lo.x + hi.x) & ~63u) | (uint32_t)lane;
-            key[1] = (ord_u32(lo.y + hi.y) & ~63u) | (uint32_t)lane;
-            key[2] = (ord_u32(lo.z + hi.z) & ~63u) | (uint32_t)lane;
+            // centroids (doubled) as ordered integers; below the largest integer, which only a NaN can be
+            key[0] = min(ord_u32(lo.x + hi.x), 0xFFFFFFFEu);
+            key[1] = min(ord_u32(lo.y + hi.y), 0xFFFFFFFEu);
+            key[2] = min(ord_u32(lo.z + hi.z), 0xFFFFFFFEu);
         }
-        // rank of each primitive along each axis: the keys below its own
+        // rank of each primitive along each axis: the keys below its own, and equal ones of lanes below.
+        // (Keys with the lane in their low 6 bits instead left 18 bits of the centroid: a cluster of
+        // extent 0.1 at a coordinate of 10,000 fell into one or two values, its order that of the lanes.)
         uint32_t rank[3] = {0u, 0u, 0u}, ord[3];
         for (int j = 0; j < m; j++)
             for (int ax = 0; ax < 3; ax++)
-                rank[ax] += (uint32_t)__builtin_amdgcn_readlane((int)key[ax], j) < key[ax] ? 1u : 0u;
+                rank[ax] += (uint32_t)__builtin_amdgcn_readlane((int)key[ax], j) < key[ax] + (j < lane ? 1u : 0u) ? 1u : 0u;
         for (int ax = 0; ax < 3; ax++) {
             s_ord[mine ? rank[ax] : (uint32_t)lane] = (uint32_t)lane;
             wave_sync();

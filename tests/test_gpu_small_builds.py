@@ -70,3 +70,33 @@ def test_sah_clusters_of_hard_geometry(device, stream, kind, n):
     scene, f = ob.single_mesh_scene(verts, tris), lc.rays_as_floats(rays)
     compare_closest(host.trace_closest(device, stream, accel, rays), scene.trace_closest2(f), rays)
     compare_any(host.trace_any(device, stream, accel, rays), scene.trace_any(f))
+
+
+@pytest.mark.parametrize("n,extent", ((64, 0.125), (64, 0.5), (1000, 0.25)))
+def test_sah_clusters_far_from_the_origin(device, stream, n, extent):
+    """The same geometry near the origin and at a coordinate of 10,000, its vertices multiples of 2^-9,
+    so that positions, centroids and extents are exact in both places: the trees are equally good (rays
+    visit as many nodes and test as many triangles) however close the centroids lie for their size."""
+    rng = np.random.default_rng(n)
+    grid = int(extent * 512)
+    at = rng.integers(0, grid, (n, 1, 3)) + rng.integers(-2, 3, (n, 3, 3))
+    rays = np.zeros(20000, lc.RAY_DTYPE)
+    origin = rng.integers(-grid, 2 * grid, (len(rays), 3))
+    target = rng.uniform(0, extent, (len(rays), 3))
+    rays["direction"] = (target - origin / 512.0).astype(np.float32)
+    rays["t_min"], rays["t_max"] = 0.0, 1e30
+    work = []
+    for offset in (0, 10000):
+        v = np.zeros((3 * n, 4), np.float32)
+        v[:, :3] = (at / 512.0 + offset).reshape(-1, 3)
+        mesh = host.mesh_from_arrays(device, stream, v, np.arange(3 * n, dtype=np.uint32).reshape(-1, 3))
+        accel = device.create_accel()
+        accel.emplace_back(mesh)
+        stream << accel.build()
+        rays["origin"] = (origin / 512.0 + offset).astype(np.float32)
+        work.append(accel.trace_count(stream, host.upload(device, stream, rays), len(rays)))
+        print(f"[far] {n} triangles over {extent} at {offset}: nodes and triangles {work[-1]}", flush=True)
+        errs = mesh.validate(stream)
+        assert not any(errs.values()), errs
+    near, far = np.array(work, np.float64)
+    assert (far <= 1.02 * near).all(), work
