@@ -96,8 +96,8 @@ struct TraceParams {
     uint32_t *ray_counter;
     const uint32_t *order; // optional: queue indices in traversal order (sorted queue), else identity
     Geometry geo;
-    uint2 *spill;
-    uint32_t spill_depth; // spill entries per lane
+    uint2 *spill;         // TraceGrid::spill_areas areas of spill_depth entries
+    uint32_t spill_depth;
     int steps;            // traversal steps between ray refills
     unsigned long long *stats; // [nodes visited, triangles tested] when counting
     uint32_t *error;
@@ -302,6 +302,13 @@ struct TraceGrid {
     int grid;
     uint32_t lanes;
     bool octets;
+    // Stack spill areas of the launch (of `block` lanes per workgroup): one for each ray a wave can take.
+    // Never more for fewer rays, whatever the forms: a captured launch has to fit the memory that an
+    // earlier, larger one left.
+    uint64_t spill_areas(int block) const {
+        const uint64_t waves = octets ? (uint64_t)grid : (uint64_t)grid * (uint64_t)(block / 64);
+        return waves * (lanes != 0u ? lanes : 64u);
+    }
 };
 TraceGrid trace_grid(uint64_t count, int block, int blocks_per_cu, int cu_count, bool octets);
 hipError_t trace_launch(const TraceParams &P, hipStream_t stream, bool any, bool two, bool count, int grid, int block,

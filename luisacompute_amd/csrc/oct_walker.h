@@ -50,9 +50,10 @@ struct OctWalker {
 
     static constexpr uint32_t kWorld = 0xFFFFFFFFu;
 
-    // as Walker: the host sizes spill_depth (from at most 24 LDS entries) by the built depths
+    // As Walker: the host sizes spill_depth (from at most 24 LDS entries) by the built depths. One area
+    // per ray (TraceGrid::spill_areas); queues counted on the device have the areas of 64 lanes per wave.
     __device__ __forceinline__ uint2 *spill_at(const TraceParams &P, int e) const {
-        return P.spill + ((uint64_t)blockIdx.x * 64u + 8u * group) * P.spill_depth + e;
+        return P.spill + ((uint64_t)blockIdx.x * (P.octets ? P.lanes : 8u) + group) * P.spill_depth + e;
     }
     __device__ __forceinline__ void push(const TraceParams &P, uint2 e) {
         if (sp < kOctStack) stk[sp][group] = e; // the eight lanes store the same value

@@ -838,8 +838,8 @@ static int run_wave(Device *dev, hipStream_t s, Workspace &W, const PtBinding &B
     const uint32_t sd_c = Bd.stack_need > (uint32_t)cc.slds ? Bd.stack_need - cc.slds : 0u;
     const uint32_t sd_a = Bd.stack_need > (uint32_t)ca.slds ? Bd.stack_need - ca.slds : 0u;
     {
-        const size_t need = std::max<size_t>({16, (size_t)grid_c * cc.block * sd_c * sizeof(uint2),
-                                              (size_t)grid_a * ca.block * sd_a * sizeof(uint2)});
+        const size_t need = std::max<size_t>({16, tg_c.spill_areas(cc.block) * sd_c * sizeof(uint2),
+                                              tg_a.spill_areas(ca.block) * sd_a * sizeof(uint2)});
         void *sp = W.spill;
         size_t have = W.spill_bytes;
         PT_TRY(grow(sp, have, need, W.generation));

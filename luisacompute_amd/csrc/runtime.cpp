@@ -1697,7 +1697,7 @@ static int trace_launch_batches(Device *dev, Accel *a, hipStream_t s, const lc_h
     P.octets = tg.octets ? 1u : 0u;
     P.simds = count_ptr ? 4u * (uint32_t)std::max(1, dev->cu_count) : 0u;
     P.spill_depth = stack_need > (uint32_t)cfg.slds ? stack_need - (uint32_t)cfg.slds : 0u;
-    size_t spill_bytes = (size_t)grid * cfg.block * P.spill_depth * sizeof(uint2);
+    const size_t spill_bytes = tg.spill_areas(cfg.block) * P.spill_depth * sizeof(uint2);
     StreamScratch *S = stream_scratch(dev, s);
     if (!S) return fail(LC_HIP_ERROR_OUT_OF_MEMORY, "stream scratch");
     LC_HIP_GROW((S, s, S->spill, S->spill_bytes, spill_bytes));
@@ -1939,7 +1939,6 @@ int lc_hip_accel_trace_closest_noalloc(uint64_t device, uint64_t stream, uint64_
     const TraceConfig &cfg = dev->cfg[0];
     const int bpc = cfg.blocks_per_cu > 0 ? cfg.blocks_per_cu : trace_blocks_per_cu(false, two, false, cfg.block, cfg.slds);
     TraceGrid tg = trace_grid(ray_count, cfg.block, bpc, dev->cu_count, true);
-    uint64_t grid = (uint64_t)tg.grid;
     P.spill_depth = stack_need > (uint32_t)cfg.slds ? stack_need - (uint32_t)cfg.slds : 0u;
     const size_t spill_per_block = (size_t)cfg.block * P.spill_depth * sizeof(uint2);
     const size_t spill_cap = kNoAllocScratchBytes - kNoAllocWordsBytes;
@@ -1947,11 +1946,8 @@ int lc_hip_accel_trace_closest_noalloc(uint64_t device, uint64_t stream, uint64_
         return fail(LC_HIP_ERROR_UNSUPPORTED, "traversal stacks of one workgroup need " + std::to_string(spill_per_block) +
                                                   " spill bytes, more than the no-allocation scratch holds (" +
                                                   std::to_string(spill_cap) + ")");
-    if (spill_per_block && grid > spill_cap / spill_per_block) { // a smaller grid: waves claim slots as they go
-        grid = spill_cap / spill_per_block;
-        tg.lanes = 0u;
-        tg.octets = false;
-    }
+    if (tg.spill_areas(cfg.block) * P.spill_depth * sizeof(uint2) > spill_cap) // a smaller grid: waves claim slots as they go
+        tg = TraceGrid{(int)std::min<uint64_t>((uint64_t)bpc * std::max(1, dev->cu_count), spill_cap / spill_per_block), 0u, false};
     P.lanes = tg.lanes;
     P.octets = tg.octets ? 1u : 0u;
     static_assert(576 + 2 * sizeof(unsigned long long) <= kNoAllocWordsBytes, "no-allocation words");
@@ -1963,7 +1959,7 @@ int lc_hip_accel_trace_closest_noalloc(uint64_t device, uint64_t stream, uint64_
     set_step_policy(P, cfg);
     P.fetch_chunk = cfg.fetch_chunk;
     P.fetch_segments = cfg.fetch_segments;
-    const hipError_t e = trace_launch(P, s, false, two, false, (int)grid, cfg.block, cfg.slds);
+    const hipError_t e = trace_launch(P, s, false, two, false, tg.grid, cfg.block, cfg.slds);
     if (e != hipSuccess) return hip_fail(e, "trace launch");
     return LC_HIP_OK;
 }
@@ -2024,13 +2020,12 @@ int lc_hip_accel_query(uint64_t device, uint64_t stream, uint64_t accel, uint64_
     const bool first = P.first != 0u;
     const TraceConfig &cfg = dev->cfg[first ? 1 : 0];
     const int block = query_block(first), bpc = query_blocks_per_cu(first), cus = std::max(1, dev->cu_count);
-    int grid;
+    TraceGrid tg;
     if (first) {
         const uint64_t want = ((uint64_t)ray_count + block - 1) / block;
-        grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)bpc * cus, want));
+        tg = TraceGrid{(int)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)bpc * cus, want)), 0u, false};
     } else {
-        const TraceGrid tg = trace_grid(ray_count, block, bpc, cus, false);
-        grid = tg.grid;
+        tg = trace_grid(ray_count, block, bpc, cus, false);
         P.lanes = tg.lanes;
     }
     set_step_policy(P, cfg);
@@ -2040,7 +2035,7 @@ int lc_hip_accel_query(uint64_t device, uint64_t stream, uint64_t accel, uint64_
     P.spill_depth = stack_need > slds ? stack_need - slds : 0u;
     StreamScratch *S = stream_scratch(dev, s);
     if (!S) return fail(LC_HIP_ERROR_OUT_OF_MEMORY, "stream scratch");
-    LC_HIP_GROW((S, s, S->spill, S->spill_bytes, (size_t)grid * block * P.spill_depth * sizeof(uint2)));
+    LC_HIP_GROW((S, s, S->spill, S->spill_bytes, tg.spill_areas(block) * P.spill_depth * sizeof(uint2)));
     P.spill = static_cast<uint2 *>(S->spill);
     P.error = S->error;
     P.ray_counter = S->ray_counter;
@@ -2059,7 +2054,7 @@ int lc_hip_accel_query(uint64_t device, uint64_t stream, uint64_t accel, uint64_
         hipError_t e = ray_sort(s, bt, ray_count, nullptr, a->world_bounds, S->sort, S->sort_bytes, &P.order);
         if (e != hipSuccess) return hip_fail(e, "query ray sort");
     }
-    hipError_t e = query_launch(P, s, grid);
+    hipError_t e = query_launch(P, s, tg.grid);
     if (e != hipSuccess) return hip_fail(e, "query launch");
     return LC_HIP_OK;
 }

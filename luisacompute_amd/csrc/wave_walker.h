@@ -129,10 +129,14 @@ struct WaveWalker {
         batch = ray = 0u;
     }
 
-    // This lane's spill entry k. As in Walker the host sizes spill_depth from the built depths; the
-    // checks only guard memory.
+    // This lane's spill entry k (TraceGrid::spill_areas; traces that count nothing take 64 rays per wave,
+    // or eight lanes per ray). As in Walker the host sizes spill_depth from the built depths; the checks
+    // only guard memory.
     __device__ __forceinline__ uint2 *spill_at(const Params &P, int k) const {
-        return P.spill + ((uint64_t)blockIdx.x * BLOCK + tid) * P.spill_depth + k;
+        uint64_t area = (uint64_t)blockIdx.x * BLOCK + tid;
+        if ((kQuery || COUNT) && P.lanes != 0u)
+            area = ((uint64_t)blockIdx.x * (BLOCK / 64) + (tid >> 6)) * P.lanes + lane;
+        return P.spill + area * P.spill_depth + k;
     }
     __device__ __forceinline__ void push(const Params &P, uint2 e) {
         if (sp < SLDS) sh->stk[sp][tid] = e;
