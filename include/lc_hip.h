@@ -599,7 +599,10 @@ int lc_hip_trace_set_config(uint64_t device, int kind, int block, int lds_stack,
 int lc_hip_trace_get_config(uint64_t device, int kind, int *block, int *lds_stack, int *steps, int *blocks_per_cu);
 /* 1 = traverse rays in the order of a sort by (origin Morton code in the scene box, direction
    octant) so neighbouring lanes share subtrees; results still land in each ray's own slot.
-   Applies to plain, batched, device-counted (indirect) and captured traces and to ray queries. */
+   Applies to plain, batched, device-counted (indirect) and captured traces and to ray queries where
+   it pays: launches of at least 262,144 rays (device-counted ones: of that capacity), and, over two or
+   more instances, scenes whose points lie in 1.5 instance boxes or more on average (small instances
+   apart from the rest do not count). */
 int lc_hip_trace_set_ray_sort(uint64_t device, int kind, int enable);
 int lc_hip_trace_get_ray_sort(uint64_t device, int kind, int *enable);
 /* How a persistent trace launch hands out queue slots: a wave claims `chunk` slots per atomic

@@ -518,7 +518,8 @@ class Device:
         return dict(block=v[0].value, lds_stack=v[1].value, steps=v[2].value, blocks_per_cu=v[3].value)
 
     def set_ray_sort(self, kind, enable):
-        """Traverse rays in sorted-queue order (origin Morton code, direction octant)."""
+        """Traverse rays in sorted-queue order (origin Morton code, direction octant): launches of at least
+        262,144 rays and, over several instances, scenes whose points lie in 1.5 instance boxes on average."""
         _check(lib().lc_hip_trace_set_ray_sort(self.handle, 1 if kind == "any" else 0, 1 if enable else 0), "ray sort")
 
     def ray_sort(self, kind):

@@ -29,7 +29,7 @@ HIP_FLAGS = [f"--offload-arch={ARCH}", "-fgpu-flush-denormals-to-zero",
 
 SOURCES = ["bvh_build.hip", "trace.hip", "radix.hip", "raysort.hip", "pathtracer.hip", "instances.hip", "query.hip", "serve.cpp", "runtime.cpp",
            "workload.cpp", "shader.cpp", "lc_api.cpp"]
-HEADERS = ["lc_hip_bvh.h", "lc_hip_internal.h", "traverse.h", "wave_walker.h", "oct_walker.h", "ray_query.h", "lc_hip_rtx.h", "lc_hip_device.h"]
+HEADERS = ["lc_hip_bvh.h", "lc_hip_internal.h", "box_overlap.h", "traverse.h", "wave_walker.h", "oct_walker.h", "ray_query.h", "lc_hip_rtx.h", "lc_hip_device.h"]
 # The device library of run-time shaders: embedded into the library as in-memory headers for hiprtc.
 DEVICE_HEADERS = ["lc_hip_device.h", "lc_hip_bvh.h", "lc_hip_rtx.h", "ray_query.h", "traverse.h"]
 

@@ -142,10 +142,11 @@ hipError_t exclusive_scan_u32_counted(hipStream_t stream, const uint32_t *in, ui
 // itself got faster); at 131,072 281 us sorted against 241, at 524,288 565 against 668.
 constexpr uint64_t kSortMinRays = 1u << 18;
 // Two-level scenes whose rays' queues are sorted: those where a point lies in this many instance boxes
-// on average. Where instances lie apart, few of a ray's fetches are those of its neighbours in origin
-// and direction (2.1M rays, unsorted / sorted: 2 overlapping soups of 1M triangles 3,763 / 3,145 us, 8
-// of them 5,825 / 5,075; 64 side by side 3,046 / 3,283, 1,000 spheres side by side 1,626 / 1,688; 1,024
-// scattered instances 757 / 885).
+// on average (box_overlap.h; small instances far away change nothing). Where instances lie apart, few of a
+// ray's fetches are those of its neighbours in origin and direction (2.1M rays, unsorted / sorted: 2
+// overlapping soups of 1M triangles 2,750 / 2,530 us, and with a small instance at 9 times the scene's
+// size 2,759 / 2,527; shifted by half 2,340 / 2,267; 100 scattered groups of 3 overlapping soups 1,255 /
+// 1,580; 1,024 scattered instances 2,368 / 2,660; 64 side by side 3,046 / 3,283).
 constexpr double kSortMinOverlap = 1.5;
 // count_ptr (device word, may be null): only the first min(*count_ptr, n) rays are sorted.
 size_t ray_sort_scratch_bytes(uint32_t n);
@@ -513,7 +514,7 @@ struct Accel {
     bool built = false;
     uint32_t max_blas_depth = 0;
     float world_bounds[6] = {0, 0, 0, 0, 0, 0}; // union of instance world boxes (ray-sort keys)
-    double box_overlap = 0.0; // instance boxes that cover a point of the scene box on average (last build)
+    double box_overlap = 0.0; // instance boxes that a point of the scene lies in on average (last build of two or more)
     // device-side instance table for the in-kernel instance ops (state[count] is the
     // out-of-range-index flag word); written at every build, folded back into `inst` before the
     // next build when instance writes were issued

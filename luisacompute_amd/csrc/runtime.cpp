@@ -17,6 +17,7 @@
 #include <memory>
 #include <string>
 
+#include "box_overlap.h"
 #include "lc_hip_internal.h"
 
 using namespace lchip;
@@ -1426,7 +1427,6 @@ int lc_hip_accel_build(uint64_t device, uint64_t stream, uint64_t accel, uint32_
     // world boxes of instances: 8 transformed BLAS-box corners, padded by a relative epsilon
     float *boxes = reinterpret_cast<float *>(a->stage + off_box);
     {
-        double volumes = 0.0;
         float wlo[3] = {3e38f, 3e38f, 3e38f}, whi[3] = {-3e38f, -3e38f, -3e38f};
         for (uint32_t i = 0; i < instance_count; i++) {
             float lo[3] = {3e38f, 3e38f, 3e38f}, hi[3] = {-3e38f, -3e38f, -3e38f};
@@ -1445,7 +1445,6 @@ int lc_hip_accel_build(uint64_t device, uint64_t stream, uint64_t accel, uint32_
                     wlo[k] = std::min(wlo[k], lo[k]);
                     whi[k] = std::max(whi[k], hi[k]);
                 }
-                volumes += ((double)hi[0] - lo[0]) * ((double)hi[1] - lo[1]) * ((double)hi[2] - lo[2]);
             } else {
                 // no geometry: a degenerate box far outside any scene (never entered: blas_nodes == 0)
                 for (int k = 0; k < 3; k++) { lo[k] = hi[k] = 3e38f; }
@@ -1458,9 +1457,6 @@ int lc_hip_accel_build(uint64_t device, uint64_t stream, uint64_t accel, uint32_
             a->world_bounds[k] = wlo[k] <= whi[k] ? wlo[k] : 0.0f;
             a->world_bounds[3 + k] = wlo[k] <= whi[k] ? whi[k] : 0.0f;
         }
-        double volume = 1.0;
-        for (int k = 0; k < 3; k++) volume *= (double)a->world_bounds[3 + k] - a->world_bounds[k];
-        a->box_overlap = volume > 0.0 ? volumes / volume : 0.0;
     }
     if (instance_count > 1) {
         p = a->boxes; cap = a->box_cap;
@@ -1496,6 +1492,7 @@ int lc_hip_accel_build(uint64_t device, uint64_t stream, uint64_t accel, uint32_
         }
         LC_HIP_TRY(hipEventRecord(a->tlas_ready, s));
         a->tlas_valid = true;
+        a->box_overlap = box_overlap(boxes, instance_count); // while the GPU builds
     } else {
         const int rc = upload_tables(0);
         if (rc != LC_HIP_OK) return rc;
