@@ -231,8 +231,8 @@ __global__ __launch_bounds__(BLOCK) void k_pt_mega(const PtScene S, const Geomet
     __shared__ uint2 stk[SLDS][BLOCK];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint64_t glane = (uint64_t)blockIdx.x * BLOCK + tid;
-    trav::Walker<false, TWO, false, BLOCK, SLDS> Wc;
-    trav::Walker<true, TWO, false, BLOCK, SLDS> Wa;
+    trav::Walker<false, TWO, BLOCK, SLDS> Wc;
+    trav::Walker<true, TWO, BLOCK, SLDS> Wa;
     Wc.init(G, stk, tid, spill + glane * spill_depth, spill_depth, error);
     Wa.init(G, stk, tid, spill + glane * spill_depth, spill_depth, error);
     const uint32_t tiles_x = (S.width + 7u) / 8u, tiles = tiles_x * ((S.height + 7u) / 8u);

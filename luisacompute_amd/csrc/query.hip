@@ -148,7 +148,7 @@ __global__ __launch_bounds__(kQueryBlock) void k_query(const QueryParams P) {
             if (!active && !exhausted) {
                 if (my < count) {
                     ray = P.order ? P.order[my] : my;
-                    W.start(P.geo, P.rays[2 * (uint64_t)ray], P.rays[2 * (uint64_t)ray + 1], P.mask, P.first != 0u);
+                    W.start(P.geo, P.rays[2 * (uint64_t)ray], P.rays[2 * (uint64_t)ray + 1], P.mask, true);
                     active = true;
                 } else if (drained) {
                     exhausted = true;

@@ -19,8 +19,9 @@
 // of the visiting order; ties at equal t go to the smaller (instance, primitive) pair, as in
 // trace_closest.
 //
-// The walk is one ray per lane. Nearest-commit queries take wave-uniform steps (leaf records or
-// nodes, as the closest-hit walker of traverse.h); first-commit queries let each lane finish a
+// The walk is one ray per lane (run-time shaders, and the library's first-commit queries; its
+// nearest-commit ones walk as wave_walker.h does). Nearest-commit queries take wave-uniform steps (leaf
+// records or nodes, as the closest-hit walker of traverse.h); first-commit queries let each lane finish a
 // node's leaf records before its next node (a commit ends them). The walk is resumable
 // (QueryWalker::run advances a bounded number of steps), so persistent kernels refill the lanes
 // whose query finished, as the trace kernel does. Procedural BLASes hold one

@@ -1,5 +1,6 @@
-// traverse.h -- per-ray BVH8 traversal state machine shared by the persistent trace kernel
-// (trace.hip) and the path-tracing kernels (pathtracer.hip).
+// traverse.h -- BVH8 traversal: the node and triangle tests of every walker, and the per-lane walker of
+// the path tracer's megakernel (pathtracer.hip). Trace launches walk as wave_walker.h and oct_walker.h
+// do, first-commit queries and run-time shaders as ray_query.h does.
 //
 // Observable semantics follow the CPU backend's AccelImpl::trace_closest / trace_any
 // (src/rust/luisa_compute_backend_impl/src/cpu/accel.rs:449-535):
@@ -202,18 +203,6 @@ __device__ __forceinline__ void load_node(const WideNode *nodes, uint32_t idx, u
 constexpr uint32_t kInstGroup = 0x80000000u; // stack entry tag: remaining instances of a TLAS leaf
 constexpr uint32_t kTriGroup = 0x40000000u;  // stack entry tag: postponed triangles of a BLAS node
 
-// Wave-uniform step choice (speculative traversal, Aila and Laine, "Understanding the Efficiency
-// of Ray Traversal on GPUs", HPG 2009): a step tests triangles only when at least
-// kTriQuarters/4 of the wave's live lanes hold triangles; otherwise it visits nodes, and lanes
-// that hold triangles but still have a node group visit a node too (their triangles wait, and
-// are pushed as a tagged stack entry if the new node brings leaves of its own). Each step then
-// runs one of the two code paths instead of both.
-constexpr bool kSpeculate = true;      // closest hit
-constexpr bool kSpeculateAny = false;  // any hit (a lane tests its triangles first: a hit ends it)
-constexpr bool kSpeculateNodes = true; // triangle-holding lanes visit nodes in node steps
-constexpr int kTriQuarters = 2;
-constexpr int kTriQuartersAny = 2;
-
 // (t, inst, prim) is nearer than the current best, or as near with a smaller (inst, prim) key.
 __device__ __forceinline__ bool nearer(float t, uint32_t inst, uint32_t prim, float t_best, uint32_t b_inst,
                                        uint32_t b_prim) {
@@ -221,11 +210,10 @@ __device__ __forceinline__ bool nearer(float t, uint32_t inst, uint32_t prim, fl
     return inst != b_inst ? inst < b_inst : prim < b_prim;
 }
 
-// One ray's traversal (the path tracer's megakernel; trace launches use the walkers of wave_walker.h and
-// oct_walker.h). ANY: stop at the first hit; TWO: TLAS + BLAS (otherwise the single
-// instance of G); COUNT: count node visits and triangle tests. The stack's LDS part is the
-// column `tid` of an [SLDS][BLOCK] array; entries beyond SLDS go to `spill`.
-template<bool ANY, bool TWO, bool COUNT, int BLOCK, int SLDS>
+// One ray's traversal (the path tracer's megakernel). ANY: stop at the first hit; TWO: TLAS + BLAS
+// (otherwise the single instance of G). The stack's LDS part is the column `tid` of an [SLDS][BLOCK]
+// array; entries beyond SLDS go to `spill`.
+template<bool ANY, bool TWO, int BLOCK, int SLDS>
 struct Walker {
     uint2 (*stk)[BLOCK];
     uint32_t tid;
@@ -247,14 +235,11 @@ struct Walker {
     uint32_t cur_inst;
     const WideNode *nodes;
     const TriRecord *tris;
-    // counting form only: node visits, triangle tests, loop iterations this lane spent live in
-    // run(), and wave iterations (counted by the wave's first live lane)
-    uint64_t n_nodes, n_tris, n_live, n_wave;
 
     __device__ __forceinline__ void init(const Geometry &G, uint2 (*s)[BLOCK], uint32_t t, uint2 *spill_lane,
                                          uint32_t depth, uint32_t *err) {
         stk = s; tid = t; spill = spill_lane; spill_depth = depth; error = err;
-        sp = 0; n_nodes = 0; n_tris = 0; n_live = 0; n_wave = 0;
+        sp = 0;
         // single-instance form: the BLAS pointers never change (kept uniform)
         in_blas = !TWO;
         nodes = TWO ? G.tlas_nodes : G.blas_nodes;
@@ -305,31 +290,24 @@ struct Walker {
         }
     }
 
-    // Runs up to `steps` traversal steps; true when the ray is finished. Closest hit takes a
-    // triangle step when 4 x (lanes holding triangles) >= tri_quarters x (live lanes) (0: the
-    // default kTriQuarters); with
-    // refill_below > 0 the wave stops early (false for every live lane) once fewer lanes than that
-    // hold a ray, so that the caller can refill the idle ones (can_refill: slots are left).
-    __device__ __forceinline__ bool run(const Geometry &G, int steps, uint32_t tri_quarters = kTriQuarters,
-                                        uint32_t refill_below = 0u, bool can_refill = false) {
-        constexpr bool SPEC = ANY ? kSpeculateAny : kSpeculate;
+    // Runs up to `steps` traversal steps; true when the ray is finished. Closest hit takes wave-uniform
+    // steps (speculative traversal, Aila and Laine, "Understanding the Efficiency of Ray Traversal on
+    // GPUs", HPG 2009): a step tests triangles when at least half of the wave's live lanes hold some;
+    // otherwise it visits nodes, and lanes that hold triangles but still have a node group visit a node
+    // too (their triangles wait, and are pushed as a tagged stack entry if the new node brings leaves of
+    // its own). Each step then runs one of the two code paths instead of both. Any hit: a lane tests its
+    // triangles first, as a hit ends it.
+    __device__ __forceinline__ bool run(const Geometry &G, int steps) {
+        constexpr bool SPEC = !ANY;
         for (int it = 0; it < steps; it++) {
-            if (COUNT) {
-                n_live++;
-                if (__lane_id() == (uint32_t)__ffsll((long long)__ballot(1)) - 1u) n_wave++;
-            }
-            if (refill_below != 0u && can_refill && it > 0 && (uint32_t)__popcll(__ballot(1)) < refill_below)
-                return false;
             const float tcull = ANY ? tmax : fminf(tmax, t_best);
             bool tri_step = t_mask != 0u;
             if (SPEC) {
                 if (t_mask == 0u && (g_mask & 0xFFu) == 0u && sp == 0) return true;
                 const uint32_t n_live = (uint32_t)__popcll(__ballot(1));
                 const uint32_t n_tri = (uint32_t)__popcll(__ballot(t_mask != 0u));
-                const uint32_t tq = ANY ? (uint32_t)kTriQuartersAny : (tri_quarters ? tri_quarters : (uint32_t)kTriQuarters);
-                tri_step = 4u * n_tri >= tq * n_live;
+                tri_step = 2u * n_tri >= n_live;
                 if (tri_step && t_mask == 0u) continue;
-                if (!tri_step && !kSpeculateNodes && t_mask != 0u) continue;
             }
             if (tri_step) {
                 const uint32_t b = (uint32_t)__builtin_ctz(t_mask);
@@ -337,7 +315,6 @@ struct Walker {
                 if (!TWO || in_blas) {
                     const float4 *tr = reinterpret_cast<const float4 *>(tris + t_base + b);
                     const float4 a = tr[0], bb = tr[1], c = tr[2];
-                    if (COUNT) n_tris++;
                     float t, u, v;
                     if (wt_intersect(R, a, bb, c, tmin, tmax, t, u, v)) {
                         if (ANY) { any_hit = true; return true; }
@@ -417,7 +394,6 @@ struct Walker {
             g_mask = 0u;
             uint4 w0, w1, w2, w3, w4;
             load_node(nodes, node, w0, w1, w2, w3, w4);
-            if (COUNT) n_nodes++;
             const uint32_t hits = intersect_node(R, w0, w1, w2, w3, w4, tmin, tcull);
             const uint32_t nim = w0.w >> 24;
             g_base = w1.x;

@@ -106,7 +106,7 @@ struct WaveWalker {
     uint32_t cur_flags;    // queries: its InstanceRecord flags
     const WideNode *nodes;
     const TriRecord *tris;
-    uint64_t n_nodes, n_tris, n_live, n_wave; // counting form only, as in Walker
+    uint64_t n_nodes, n_tris, n_live, n_wave; // counting form only: node visits, triangle tests, lane and wave steps (account)
 
     static constexpr uint32_t kWorld = 0xFFFFFFFFu;
     __device__ __forceinline__ bool in_blas() const { return !TWO || cur_inst != kWorld; }
@@ -448,7 +448,7 @@ struct WaveWalker {
     // Returns when no lane has work left, or, with P.refill_below > 0 and rays to hand out
     // (can_refill), once fewer lanes than that are busy.
     __device__ __forceinline__ void run(const Params &P, bool active, bool can_refill) {
-        const uint32_t full = 16u * (P.tri_quarters ? P.tri_quarters : (uint32_t)kTriQuarters);
+        const uint32_t full = 16u * P.tri_quarters; // 1..4 (set_step_policy)
         const uint32_t refill_below = can_refill ? P.refill_below : 0u;
         for (int it = 0; it < P.steps; it++) {
             const bool work = active && node_work();
