@@ -605,7 +605,8 @@ class WavefrontPathTracer:
     into a graph (Stream.capture) and replayed for the following waves; the first sample of a wave
     advances in device memory, so every replay is the same launch sequence. sort_queues: the
     traces sort their queues (origin cell, direction octant; the library's radix sort, which
-    reads the device-side count) before traversal; the image is the same either way."""
+    reads the device-side count) before traversal where Device.set_ray_sort says that sorting
+    pays; the image is the same either way."""
 
     KERNELS = ("wf_clear", "wf_camera", "wf_reset", "wf_shade", "wf_resolve", "wf_accumulate", "wf_finish")
 

@@ -1,5 +1,7 @@
 """GPU tests of nearest-commit queries (query.hip, k_query_nearest) around the sizes at which a launch
-changes its form, over one instance (triangles or boxes, no TLAS) and several, against the oracle."""
+changes its form, over one instance (triangles or boxes, no TLAS) and several, against the oracle: few
+queries per wave, one for each lane, and (from 327,681 on) waves that claim them and refill their lanes,
+in queue order and (from 262,144 on) sorted."""
 import numpy as np
 import pytest
 
@@ -41,3 +43,42 @@ def test_query_sizes(device, stream, kind, n):
     for mask in (0xFF, 0x02):
         g = host.query(device, stream, accel, rays, mask, **POLICY)
         compare_query(g, sc.query(rays, mask, **POLICY), sc, rays, mask=mask, **POLICY)
+
+
+@pytest.fixture(scope="module", params=("triangles", "both"))
+def large(device, stream, request):
+    """The scene, queries and their answers from launches of at most 50,000, in which each query has a
+    lane and no lane a second one."""
+    accel, sc = _scene(device, stream, request.param)
+    saved = device.ray_sort("closest")
+    rays = lc.rays_as_floats(lc.rays_box_sphere(420001, initseq=78, lo=-2.0, hi=3.0))
+    device.set_ray_sort("closest", False)
+    want = np.concatenate([host.query(device, stream, accel, rays[k:k + 50000], 0xFF, **POLICY)
+                           for k in range(0, len(rays), 50000)])
+    some = np.random.default_rng(79).choice(len(rays), 5000, replace=False)
+    compare_query(want[some], sc.query(rays[some], 0xFF, **POLICY), sc, rays[some], **POLICY)
+    if request.param == "both":  # the instances overlap enough to be sorted (262,144 rays have a lane each)
+        rb, steps = host.upload(device, stream, host.as_rays(rays[:262144])), []
+        for on in (False, True):
+            device.set_ray_sort("closest", on)
+            steps.append(accel.trace_steps(stream, rb, 262144).wave_steps)
+        assert steps[0] != steps[1]
+    device.set_ray_sort("closest", saved)
+    return accel, rays, want
+
+
+@pytest.mark.parametrize("sort", (False, True))
+@pytest.mark.parametrize("n", (262143, 262144, 327680, 327681, 393217, 420001))
+def test_large_queries(device, stream, large, n, sort):
+    print(f"[query] {n} sort {sort}", flush=True)
+    accel, rays, want = large
+    saved, policy = device.ray_sort("closest"), device.trace_steps("closest")
+    try:
+        device.set_ray_sort("closest", sort)
+        for tq, refill in ((3, 48), (1, 63), (4, 0)):
+            device.set_trace_steps("closest", tq, refill)
+            got = host.query(device, stream, accel, rays[:n], 0xFF, **POLICY)
+            np.testing.assert_array_equal(got.view(np.uint32), want[:n].view(np.uint32))
+    finally:
+        device.set_ray_sort("closest", saved)
+        device.set_trace_steps("closest", *policy)

@@ -73,3 +73,45 @@ def test_which_launches_sort(device, stream, sorting, kind, n, sorts):
     f = lc.rays_as_floats(rays[some])
     compare_closest(got[1][0][some], sc.trace_closest2(f), rays[some])
     compare_any(got[1][1][some], sc.trace_any(f))
+
+
+@pytest.mark.parametrize("kind", ("one", "overlapping"))
+@pytest.mark.parametrize("any_hit", (False, True), ids=("closest", "any"))
+def test_captured_sorts_follow_the_count(device, sorting, kind, any_hit):
+    """A graph of a sorted trace of a queue counted on the device replays with other counts, eager work
+    between the replays: each sorts and traces the first rays, as many as are counted then."""
+    s = device.create_stream()
+    accel, _ = _scene(device, s, kind)
+    rays = lc.rays_box_sphere(N, initseq=74, lo=-5.0, hi=25.0)
+    rb, cb = host.upload(device, s, rays), device.create_buffer(4, 1)
+    size = 1 if any_hit else 24
+    out = device.create_buffer(size, N)
+
+    def read():
+        got = np.zeros(N * size, np.uint8)
+        s << out.copy_to(got) << lc.synchronize()
+        return got.reshape(N, size)
+
+    def trace():
+        (accel.trace_any_indirect if any_hit else accel.trace_closest_indirect)(s, rb, out, cb)
+
+    sorting(False)
+    s << cb.copy_from(np.array([N], np.uint32))
+    trace()
+    want = read()
+    sorting(True)
+    assert _sorts(s, accel, rb, N, lambda on: sorting(on), any_hit)
+    sorting(True)
+    trace()  # eager first: the stream then holds the sort's working memory, without which a capture does not sort
+    np.testing.assert_array_equal(read(), want)
+    with s.capture() as cap:
+        trace()
+    sorting(False)  # the graph keeps what it recorded
+    for count in (N, 0, 1, 4096, 65537, 262144, N - 1, N + 5, 77):
+        print(f"[captured sort] {kind} any {any_hit} count {count}", flush=True)
+        s << cb.copy_from(np.array([count], np.uint32)) << out.copy_from(np.full(N * size, 0xA5, np.uint8))
+        cap.graph.launch(s)
+        got = read()
+        np.testing.assert_array_equal(got[:count], want[:count])
+        assert (got[count:] == 0xA5).all()
+        host.trace_closest(device, s, accel, rays[:1000])

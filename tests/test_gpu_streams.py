@@ -126,7 +126,7 @@ def test_two_streams_trace_concurrently():
     stream = device.create_stream()
     autotune.load_default(device)  # sorted queues: the sort scratch is in use too
     scenes = []
-    for k, (ntris, nrays) in enumerate(((1 << 16, 300000), (20000, 200000))):
+    for k, (ntris, nrays) in enumerate(((1 << 16, 400001), (20000, 420000))):  # claimed slots, sorted
         verts, tris = lc.soup(ntris, initseq=60 + k)
         accel = host.single_mesh_accel(device, stream, verts, tris)
         rays = lc.rays_box_sphere(nrays, initseq=62 + k)

@@ -114,16 +114,42 @@ def _room(device, stream):
     return room, accel, meshes, inst
 
 
+def _cover(room, accel, meshes, inst, stream):
+    """Two more instances over the whole room that no ray sees: a scene of overlapping instances, whose
+    rays are sorted, with the same image."""
+    corners = [(v[:, :3].min(0), v[:, :3].max(0)) for v, _ in room.meshes]
+    k = int(np.argmax([np.prod(hi - lo) for lo, hi in corners]))
+    lo, hi = np.min([c[0] for c in corners], 0), np.max([c[1] for c in corners], 0)
+    scale = (hi - lo) / (corners[k][1] - corners[k][0])
+    a = np.zeros((3, 4), f32)
+    a[:, :3], a[:, 3] = np.diag(scale), lo - scale * corners[k][0]
+    for _ in range(2):
+        accel.emplace_back(meshes[k], a.reshape(12), visibility_mask=0)
+        inst.append(inst[k])
+    stream << accel.build()
+
+
 @pytest.mark.parametrize("w,h,spp,max_depth,per_wave,sort", [(64, 48, 4, 8, None, False), (64, 48, 4, 8, 1, True),
-                                                              (200, 120, 5, 5, 2, True), (200, 120, 5, 5, 2, False)])
+                                                              (200, 120, 5, 5, 2, True), (200, 120, 5, 5, 2, False),
+                                                              (640, 420, 2, 5, 1, True)])
 def test_dsl_wavefront_equals_dsl_megakernel(device, w, h, spp, max_depth, per_wave, sort):
     """The wavefront form renders the megakernel's image bit for bit: eagerly, and with a wave's
     launches captured once and replayed (renders of one wave, of one sample per wave, and of
     two-sample waves with a one-sample remainder; eager work between the renders), with the
-    traces' queues sorted on the device or traced in queue order."""
+    traces' queues sorted on the device (at 640x420; smaller queues never are) or traced in queue order."""
     s = device.create_stream()
     room, accel, meshes, inst = _room(device, s)
+    if sort:
+        _cover(room, accel, meshes, inst, s)
     bind = programs.PathTracerBindings(device, s, accel, inst, room.scene())
+    if w * h >= 262144:  # smaller queues and rooms without the cover are traced in queue order
+        rb = host.upload(device, s, lc.rays_box_sphere(w * h, initseq=43, lo=-1.0, hi=1.0))
+        steps, was = [], device.ray_sort("closest")
+        for on in (False, True, False):
+            device.set_ray_sort("closest", on)
+            steps.append(accel.trace_steps(s, rb, w * h).wave_steps)
+        device.set_ray_sort("closest", was)
+        assert steps[0] == steps[2] != steps[1]
     mega = programs.path_tracer.compile(device)
     img = device.create_buffer(16, w * h)
     seq = 3 << 32
