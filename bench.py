@@ -9,8 +9,10 @@ HBM before timing starts. Prints one JSON line.
 Usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu]
 """
 import argparse
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -152,8 +154,8 @@ def bench_pathtracer(a):
     # the wavefront form written in the DSL (camera / shade / resolve kernels over queues, the
     # library's persistent trace on the device-counted queues; one sample's launches captured
     # into a graph and replayed per sample): same image as the DSL megakernel
-    # (queues traced in the order the shade kernel appended them, and sorted on the device by
-    # the library's radix sort before each trace)
+    # (with the option to sort queues on the device off and on: the room's instances lie apart, where
+    # sorting costs more than it saves, so its queues are traced as they were appended either way)
     dwf_ms = dwf_same = dwfs_ms = dwfs_same = None
     if not a.pt_no_dsl_wavefront:
         from luisacompute_amd import programs
@@ -490,7 +492,7 @@ def bench_query(a):
 
 def bench_build(a):
     """BLAS builds of the soup (16,777,216 triangles) under each hint: FAST_BUILD (LBVH, 3-triangle
-    leaves), FAST_TRACE without and with the binned-SAH refinement; `steps` timed builds each."""
+    leaves), FAST_TRACE without and with the SAH refinement; `steps` timed builds each."""
     import luisacompute_amd as lc
     from luisacompute_amd import host
     verts, tris = lc.soup(a.tris)
@@ -564,6 +566,37 @@ def cpu_baseline(verts, tris, rays_f, sample_rays, total_rays):
                    f"{sample_rays} rays ({t_trace:.2f} s, {sample_rays / t_trace / 1e6:.3f} Mrays/s); "
                    f"job time estimated as build + trace scaled to {total_rays} rays"),
     }
+
+
+TRACE_SOURCES = ("trace.hip", "wave_walker.h", "oct_walker.h", "traverse.h", "lc_hip_bvh.h")
+TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "trace_closest_soup16m_traffic.json")
+
+
+def kernel_fingerprint(sources=None, table=None):
+    """Hash of what makes the headline's traversal kernel: its sources without comments and white space,
+    the compiler flags, and the closest-hit launch configuration of the tuning table."""
+    from luisacompute_amd import autotune, build
+    if sources is None:
+        sources = [open(os.path.join(build.CSRC, n)).read() for n in TRACE_SOURCES]
+    table = autotune.load_table() if table is None else table
+    config = {k: v for k, v in sorted((table or {}).get("closest", {}).items()) if k not in ("ms", "mrays_s")}
+    code = [re.sub(r"\s+", "", re.sub(r"//[^\n]*|/\*.*?\*/", "", s, flags=re.S)) for s in sources]
+    flags = [f for f in build.COMMON + build.HIP_FLAGS if ROOT not in f]
+    return hashlib.sha256(json.dumps([code, flags, config]).encode()).hexdigest()[:16]
+
+
+def traffic_profile(fingerprint, path=TRAFFIC_PROFILE):
+    """(HBM bytes, L2 hit rate, VALU instructions) per launch of the headline's traversal kernel, from
+    rocprofv3 --pmc runs of this command: FETCH_SIZE and WRITE_SIZE, each scaled by what the counter reads
+    for a 1 GiB device copy (profiles/trace_closest_soup16m_traffic.md). None for each where the profile is
+    of another kernel than the one timed here."""
+    if not os.path.exists(path):
+        return None, None, None
+    with open(path) as f:
+        p = json.load(f)
+    if p.get("kernel_fingerprint") != fingerprint:
+        return None, None, None
+    return p["hbm_bytes_per_launch"], p["l2_hit_rate"], p["sq_counters"]["SQ_INSTS_VALU"]
 
 
 def build_hints(dev, s, mesh, rb, n_rays):
@@ -730,15 +763,7 @@ def main():
     achieved = a.rays * bytes_per_ray / (kern_ms * 1e-3) / 1e9
     floor_gbs = (a.rays * (RAY_BYTES + HIT_BYTES) + st.node_bytes + st.primitive_bytes) / (kern_ms * 1e-3) / 1e9
 
-    # HBM bytes per launch of the traversal kernel: FETCH_SIZE + WRITE_SIZE from two rocprofv3
-    # --pmc runs of this command, each scaled by what the counter reads for a 1 GiB device copy
-    # (profiles/trace_closest_soup16m_traffic.md)
-    traffic = l2_hit = None
-    tpath = os.path.join(ROOT, "profiles", "trace_closest_soup16m_traffic.json")
-    if os.path.exists(tpath):
-        with open(tpath) as f:
-            tj = json.load(f)
-        traffic, l2_hit = tj.get("hbm_bytes_per_launch"), tj.get("l2_hit_rate")
+    traffic, l2_hit, valu = traffic_profile(kernel_fingerprint())
 
     hints = build_hints(dev, s, mesh, rb, a.rays)
 
@@ -779,21 +804,22 @@ def main():
         "nodes_per_ray": round(nodes_per_ray, 3),
         "tris_per_ray": round(tris_per_ray, 3),
         "roofline": {
-            "bound": "hbm",
+            "bound": "valu_issue",
             "kernel": "k_trace<closest> (persistent wave64 traversal, sorted ray queue)",
             "kernel_ms": round(kern_ms, 3),
+            # the bytes that the node visits, triangle tests, rays and hits ask for, over the kernel's time:
+            # the L2s serve a part of them, so this is not an HBM rate (hbm_gbs is)
             "achieved": round(achieved, 2),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": traffic,
+            "hbm_gbs": traffic and round(traffic / (kern_ms * 1e-3) / 1e9, 1),
+            "valu_ginstr_s": valu and round(valu / (kern_ms * 1e-3) / 1e9, 1),
             "l2_hit_rate": l2_hit,
             "traffic_source": "profiles/trace_closest_soup16m_traffic.json: FETCH_SIZE + WRITE_SIZE of k_trace<closest> "
                               "from rocprofv3 --pmc runs of this command, scaled by a 1 GiB copy's counts"
                               if traffic is not None else None,
-            # the HBM roofline is the one priced here; the counter profile shows the kernel is
-            # limited by VALU issue (divergent lanes), not by bandwidth
-            "limiter": "valu_issue",
             # lane accounting of the counting run: of the wave iterations' lane slots, the share
             # with a ray, and the shares taking a node visit / a triangle test
             "lane_steps": {"live": round(steps.live_lane_steps / lane_slots, 4),
