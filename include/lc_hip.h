@@ -284,15 +284,17 @@ int lc_hip_radix_sort_pairs_temp_bytes(uint32_t num_items, size_t *temp_bytes);
 int lc_hip_radix_sort_pairs(uint64_t device, uint64_t stream, uint64_t temp_buffer, uint64_t keys_in,
                             uint64_t keys_out, uint64_t values_in, uint64_t values_out, uint32_t num_items,
                             int begin_bit, int end_bit, uint64_t count_buffer, size_t count_offset);
-/* Counter-mode run of the same traversal: total BVH nodes visited and triangles tested. */
+/* Counter-mode run of a trace: total BVH nodes visited and triangles tested. The same queue order and
+   hand-out as the timed trace, with one lane per ray also for launches of few rays, which otherwise take
+   eight (and visit and test a little differently, in another order). */
 int lc_hip_accel_trace_count(uint64_t device, uint64_t stream, uint64_t accel, uint64_t ray_buffer, size_t ray_offset,
                              uint32_t ray_count, uint32_t vis_mask, int any, uint64_t *nodes_visited,
                              uint64_t *triangles_tested);
 /* The same counter-mode run with its lane accounting (no reference counterpart: measurement).
-   A lane takes one traversal step per loop iteration (a node visit, a triangle test, or nothing
-   when the wave's step kind does not match what it holds); live_lane_steps counts the iterations
-   lanes spent with a ray, wave_steps the iterations waves issued (x 64 = lane slots), and
-   refill_rounds the times waves handed new rays to their idle lanes. */
+   A wave's step visits a node per lane that has one, tests a queued triangle per lane (whichever lane's
+   ray it belongs to), or moves lanes into and out of instances; live_lane_steps counts the steps in
+   which a lane's ray was unfinished or the lane tested a triangle, wave_steps the steps of waves (x 64 =
+   lane slots), and refill_rounds the times waves handed new rays to their idle lanes. */
 typedef struct lc_hip_trace_steps {
     uint64_t nodes_visited;
     uint64_t triangles_tested;

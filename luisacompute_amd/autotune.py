@@ -1,5 +1,6 @@
 """Autotuner: every launch knob of the ray-tracing path is chosen by timing the real kernels with
-HIP events on the workloads they serve, and the shipped table is this module's output file.
+HIP events on the workloads they serve. The shipped table has the form of its output; its step policy was
+set from a sweep over the soup, the instances and the room together.
 
 Stages (each on the best configuration of the stages before it):
   1. traversal, per trace kind (closest / any) on the 16.7M-triangle soup, searched jointly: block

@@ -690,11 +690,11 @@ __device__ __forceinline__ void merge_lane(Box6 &b, int lane4) {
 // Lane p of a run scores the splits after position p: area(a .. p) * n_left + area(p + 1 .. b) *
 // n_right from an inclusive prefix and suffix of the boxes in each list (merging with a lane's own
 // box again changes nothing, so the lanes at the run's ends need no guard). The run's cheapest split
-// (ties: the one nearest the middle, so that equal boxes halve) marks its right side, and the three
-// lists are partitioned stably by ballots. A level costs the same however many nodes it holds:
-// one task after another over the whole wave, scanning its primitives for 45 binned candidates, took
-// 1,016 us for 1M triangles where this takes 373, and 118 us for 5,120 where this takes 35, for trees
-// that trace alike (1M soup 1,238 and 1,236 us). LDS lane exchanges bound the large builds (12 per
+// (ties: the first at or after the middle, else the last before it, so that equal boxes halve) marks its
+// right side, and the three lists are partitioned stably by ballots. A level costs the same however many
+// nodes it holds: one task after another over the whole wave, scanning its primitives for 45 binned
+// candidates, took 1,016 us for 1M triangles where this takes 378, and 118 us for 5,120 where this takes
+// 36, for trees that trace alike (1M soup 1,238 and 1,236 us). LDS lane exchanges bound the large builds (12 per
 // doubling, list and direction), the ~8 levels one after another the small ones.
 __global__ __launch_bounds__(64) void k_sah_clusters(const uint32_t *entries, const uint32_t *count_ptr, BinaryTree bt,
                                                      uint32_t *ids, const TriRecord *prec, TriRecord *srec,

@@ -85,9 +85,10 @@ struct QueryMode {
 
 constexpr int kNearestBlock = 64;
 
-// One wave per workgroup: its LDS (6,400 B) and registers let 5 run on each SIMD. 2.1M queries over
-// 524,288 cutout triangles and as many spheres 4,905 -> 3,608 us, 5,000 queries over 1,000 of each
-// 1,207 -> 227 us (one query per lane, wave-uniform leaf and node steps, before).
+// One wave per workgroup: its LDS (6,400 B) and registers (96 VGPRs, with 5 spilled to 24 B of scratch per
+// lane) let 5 run on each SIMD. 2.1M queries over 524,288 cutout triangles and as many spheres 4,790 ->
+// 3,450 us, 5,000 queries over 1,000 of each 1,207 -> 227 us (one query per lane, wave-uniform leaf and
+// node steps, before). VALU issue bounds it: 556 G instructions/s with 52% of their lanes active.
 __global__ __launch_bounds__(kNearestBlock) __attribute__((amdgpu_waves_per_eu(5)))
 void k_query_nearest(const QueryParams P) {
     __shared__ trav::WaveShared<false, kNearestBlock, 8> shared;

@@ -228,7 +228,7 @@ void invert_affine(const float m[12], float out[12]) {
 // primitive leaves (more wide nodes, fewer triangle tests: path tracer 2.56 -> 3.28 G rays/s);
 // FAST_BUILD allows 3 (fewer nodes, 19% shorter build of 16.7M triangles).
 uint32_t leaf_size_for(uint32_t hint) { return hint == LC_HIP_ACCEL_FAST_BUILD ? 3u : 1u; }
-// Binned-SAH refinement of the radix tree's clusters for every hint but FAST_BUILD (the reference
+// Sweep-SAH refinement of the radix tree's clusters for every hint but FAST_BUILD (the reference
 // CPU backend builds Embree's high-quality SAH for FAST_TRACE, cpu/accel.rs:58-62).
 uint32_t sah_for(const Device *dev, uint32_t hint) { return hint != LC_HIP_ACCEL_FAST_BUILD && dev->sah_refine ? 1u : 0u; }
 

@@ -59,8 +59,9 @@ hipError_t noalloc_scratch_lookup(void **device_ptr) {
 // Template parameters: ANY (trace_any), TWO (TLAS + BLAS; otherwise one instance's BLAS),
 // COUNT (count node visits / triangle tests), BLOCK threads, SLDS stack entries in LDS.
 // With the 8-entry LDS stack the single-level forms fit 6 (<= 80 VGPRs) and the two-level forms 5
-// (<= 96 VGPRs) waves per SIMD without spilling; the hint keeps the register allocator there
-// (deeper LDS stacks are limited by LDS first).
+// (<= 96 VGPRs) waves per SIMD; the hint keeps the register allocator there (deeper LDS stacks are
+// limited by LDS first). None spills but the two-level closest-hit form: 7 VGPRs, and 40 B of scratch
+// per lane in all, 8 of them of the eight-lane body.
 template<bool ANY, bool TWO, bool COUNT, int BLOCK, int SLDS>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(SLDS == 8 ? (TWO ? 5 : 6) : 1)))
 void k_trace(const TraceParams P) {
@@ -70,9 +71,13 @@ void k_trace(const TraceParams P) {
     if constexpr (BLOCK == 64 && !COUNT) {
         // A queue counted on the device that turns out short: eight lanes per ray, in as many waves as
         // trace_grid would take and a second round or part of one, spread over the XCDs (the last depths of
-        // a path-traced wave, whose launches are sized for its first: closest 160 -> 50 us, any 140 -> 27).
-        // The limits, 51,200 and 81,920 rays for two levels on 256 CUs, lie within the sizes at which eight
-        // lanes per ray are faster on every scene measured (trace_grid).
+        // a 1080p wave of one sample, whose launches are sized for its first: closest 160 -> 65 us, any 140
+        // -> 32). The limits on 256 CUs, measured at them, eight lanes per ray / one (which the waves claim):
+        // any hit, one level, 98,304 rays: 171 / 263 us (soup of 1M), 210 / 346 (8M), 69 / 201 (sphere of
+        // 82k); two levels, 81,920: 206 / 324 (two overlapping soups), 154 / 302 (1,024 instances), 54 / 141
+        // (room). Closest hit, one level, 61,440: 238 / 286, 254 / 335, 69 / 207; two levels, 51,200: 222 / 356
+        // (1,024 instances), 102 / 174 (room), 304 / 353 (two overlapping soups, camera), and the one case
+        // that loses, 531 / 480 (the same, incoherent; 280 / 467 at 40,960).
         constexpr uint32_t kRays = ANY ? 16u : 10u; // per resident wave
         const uint32_t blocks = gridDim.x & ~(kFetchSegments - 1u);
         if (P.simds != 0u && count <= kRays * blocks) {
@@ -170,11 +175,13 @@ int trace_blocks_per_cu(bool any, bool two, bool count, int block, int slds) {
 // A launch whose rays all fit the lanes that can be resident hands them out once, without slot
 // counters (and without the launch that clears them).
 //  - Eight lanes per ray (k_trace_oct) while kOctWaves waves per SIMD hold every ray: 65,536 rays on
-//    256 CUs. Measured, one ray per lane against eight lanes per ray, 1 M triangles of a soup,
-//    closest hit: 1,024 rays 120 -> 70 us, 16,384 172 -> 103, 32,768 175 -> 121, 49,152 186 -> 128,
-//    65,536 185 -> 183, 98,304 188 -> 214; any hit 65,536 143 -> 114; 81,920 triangles of a
-//    sphere, 16,384 rays 85 -> 41, 65,536 100 -> 71. The eight lanes do the node decode eight times,
-//    so the form loses once the SIMDs have enough waves to be bound by VALU issue.
+//    256 CUs. Measured, one ray per lane against eight lanes per ray, incoherent closest hits: soup of
+//    1M triangles, 1,024 rays 108 -> 79 us, 16,384 160 -> 109, 49,152 190 -> 141, 65,536 196 -> 185,
+//    98,304 188 -> 214; sphere of 82k, 16,384 83 -> 43, 65,536 81 -> 55; 1,024 instances, 65,536
+//    263 -> 187; any hit, soup, 65,536 147 -> 109. Two overlapping soups lose above 45,000 rays
+//    (49,152 379 -> 401, 65,536 445 -> 452; their any hits 219 -> 165), at no more than the kernel before
+//    (548). The eight lanes do the node decode eight times, so the form loses once the SIMDs have enough
+//    waves to be bound by VALU issue.
 //  - Otherwise one ray per lane; when that leaves SIMDs without a wave, waves take fewer rays (down
 //    to kMinLanes: nearest-commit queries, and traces that count their work): a wave lasts as long
 //    as its slowest ray plus the triangle steps of the others, one step after another, each a

@@ -1,5 +1,5 @@
 """GPU: the SAH refinement of FAST_TRACE builds (radix-tree clusters of <= 64 primitives rebuilt by
-binned SAH and reordered). The refined trees pass the device-side invariant check, trace like the
+sweep SAH and reordered). The refined trees pass the device-side invariant check, trace like the
 oracle, cover every primitive once, and visit no more nodes per ray than the plain radix tree."""
 import numpy as np
 import pytest
@@ -43,7 +43,7 @@ def test_sah_tree_sound_and_exact(device, stream, ntris):
 
 
 def test_sah_coincident_centroids(device, stream):
-    """Triangles sharing one centroid (no binned split exists): split by position, still exact."""
+    """Triangles sharing one centroid (every split costs the same): split by position, still exact."""
     rng = np.random.default_rng(3)
     n = 200
     verts = np.zeros((3 * n, 4), np.float32)
